@@ -1377,82 +1377,226 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 	move_point(ppos, pi, p, s0.val(), s1.val(), s2.val(), fStep, cx, cy, cz, Lx, Ly, Lz, mwrap);
 }
 
-// Sub-wave variant: S lanes per point (64/S points per wavefront), each lane
-// testing every S-th entity of a visited leaf, partial sums folded across the
-// S lanes at the end.  A lane-per-point wavefront walks the union of its
-// lanes' paths, which costs 64 paths when the active points are scattered
-// (late in the move loop); here a wavefront walks S-lane-wide paths of 64/S
-// points.  Same arithmetic per pair as k_cover; only the order of the sums
-// differs.
+// One wavefront per point, for point sets too small (or too scattered) to fill
+// the card with a lane per point.  The walk tests 64 nodes at a time: the
+// frontier of opened nodes sits in LDS in tree order, and each round tests the
+// 2^d descendants of every frontier node, d as large as fits 64 lanes (a child
+// that passes has a parent that passes: its bounds and its largest live ball
+// lie within the parent's, and rounding is monotone, so the leaves found are
+// the pre-order walk's, in its order).  Then 64 / B leaves a round, a lane per
+// entity, with the next round's records in flight.  What bounds it is the
+// chain of dependent reads: about log2(leaves)/2 node rounds and a leaf round
+// per 64 / B leaves, against one node per round in a pre-order walk.  Against
+// that walk (16 or 64 lanes a point), a whole pass, ms: 2,048 points 20.6 ->
+// 10.7; 32,768 39.1 -> 19.4; 100,003 open, nSmooth 64 132 -> 53; 96 boxes of
+// 2,048 to 8,192 80.5 -> 48.4; 48 boxes of up to 524,288 272 -> 234.
+//
+// The sums keep the order of S lanes per point, lane j adding every S-th
+// entity of a leaf from the j-th on, leaf by leaf, the S partial sums then
+// folded by halves: a hit's term goes to the queue of its lane j = (offset in
+// the leaf) mod S' (S' = min(S, B): lanes past the leaf size add nothing), and
+// the queues are added up front to back.
+//
+// A frontier of more than WV_F nodes (very large balls) falls back to the
+// pre-order walk, its leaves taken WV_F at a time.
+#define WV_F 256
+#define WV_Q 256              // queued terms per wavefront: WV_Q / S' per lane j
+__device__ __forceinline__ void wave_lds_sync() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int MODE, bool COMP, int S>
-__global__ __launch_bounds__(SKG_TILE_T) void k_cover_sub(
+__global__ __launch_bounds__(SKG_TILE_T) void k_cover_wave(
 		float4 *__restrict__ ppos, const int *__restrict__ plist, int np,
 		const float4 *__restrict__ epos, const float4 *__restrict__ eaux, const float4 *__restrict__ eorg,
-		int ne, const float4 *__restrict__ nlo, const float4 *__restrict__ nhi,
+		const int *__restrict__ ecode, int ne, const float4 *__restrict__ nlo, const float4 *__restrict__ nhi,
 		int nLeaf2, int B, float *__restrict__ out_sum, int *__restrict__ ehit, int stamp, int *__restrict__ bthr,
 		const int *__restrict__ pbox, const DevBox *__restrict__ bt, int micro,
 		float cx, float cy, float cz, float Lx, float Ly, float Lz, const int *__restrict__ lstart,
 		const int *__restrict__ npDev, const int *__restrict__ stampDev, float *__restrict__ out_dl) {
+	constexpr int NW = SKG_TILE_T / 64;
+	__shared__ int s_fr[NW][2][WV_F];
+	__shared__ float s_q[NW][3][WV_Q];
 	if (npDev) np = *npDev;
 	if (stampDev) stamp = *stampDev;
-	const int blk = xcd_tile(blockIdx.x, gridDim.x);
-	const int gl = blk * SKG_TILE_T + threadIdx.x;
-	const int ii = gl / S, sub = gl % S;
-	const int wbase = (blk * SKG_TILE_T + (threadIdx.x & ~63)) / S;
-	if (wbase >= np) return;                      // whole wavefront past the end
-	const bool valid = ii < np;
-	const int pi = plist ? plist[valid ? ii : wbase] : (valid ? ii : wbase);
+	const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+	const int ii = uniform_int(xcd_tile(blockIdx.x, gridDim.x) * NW + wv);
+	if (ii >= np) return;                         // no workgroup barrier in this kernel
+	const int pi = plist ? plist[ii] : ii;
 	const float4 p = ppos[pi];
 	const int pb = pbox ? pbox[pi] : 0;
+	const bool dl = MODE == 0 && out_dl != nullptr;
+	const unsigned long long below = (1ull << lane) - 1ull;
+	float *qx = s_q[wv][0], *qy = s_q[wv][1], *qz = s_q[wv][2];
+	// slots per leaf in a round of 64 lanes, and the lane j of the summation order
+	const int bp = B >= 64 ? 64 : (B <= 1 ? 1 : 1 << (32 - __clz(B - 1)));
+	const int sp = min(S, bp), j = lane & (sp - 1), qcap = WV_Q / sp;
+	unsigned long long same = 0;                  // the lanes of a round that share this lane's j
+	for (int r = j; r < 64; r += sp) same |= 1ull << r;
 	Sum<COMP> s0, s1, s2;
 	s0.init(); s1.init(); s2.init();
 	float hmin = INFINITY;
-	const bool dl = MODE == 0 && out_dl != nullptr;
-	int node = valid ? 1 : 0;
-	while (node) {                                // the S lanes of a point move in lockstep
-		if (S == 64) node = uniform_int(node);    // one point per wavefront: scalar node reads
-		const float4 lo = nlo[node], hi = nhi[node];
-		const bool need = brange_has(hi.w, pb) && point_box_d2<false>(lo, hi, p.x, p.y, p.z, 0.f) < lo.w;
-		if (need && node < nLeaf2) { node = 2 * node; continue; }
-		if (need) {
-			const int2 rg = leaf_range(lstart, node - nLeaf2, B, ne);
-			for (int e = rg.x + sub; e < rg.y; e += S) {
-				cover_hit<MODE, COMP, true>(e, epos[e], eaux[e], -1, true, p, eorg, ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2,
-						dl);
+	int nq = 0;                                   // terms queued for j
+	auto drain = [&]() {
+		wave_lds_sync();
+		for (int t = 0; __any(t < nq); ++t)
+			if (t < nq) {
+				s0.add(qx[t * sp + j]);
+				if (MODE == 1 || dl) s1.add(qy[t * sp + j]);
+				if (MODE == 1) s2.add(qz[t * sp + j]);
+			}
+		wave_lds_sync();
+		nq = 0;
+	};
+	// one round's records: entity e of each lane (in: there is one)
+	struct Rec { float4 A, X; int K, e; bool in; };
+	auto fetch = [&](int e, bool in) {
+		Rec r;
+		r.e = e; r.in = in;
+		if (in) {
+			r.A = epos[e];
+			r.X = eaux[e];
+			r.K = (COMP || dl) ? ecode[e] : 13;
+		}
+		return r;
+	};
+	auto take = [&](const Rec &r) {
+		bool hit = false;
+		float tx = 0.f, ty = 0.f, tz = 0.f;
+		if (r.in) {
+			float dx = fsub(r.A.x, p.x), dy = fsub(r.A.y, p.y), dz = fsub(r.A.z, p.z);
+			const float d2 = sq3(dx, dy, dz);
+			if (d2 < r.X.x) {
+				hit = true;
+				if ((COMP || dl) && r.K != 13) {  // 9(ix+1) + 3(iy+1) + (iz+1)
+					const float4 O = eorg[r.e];
+					dx = exact_delta(O.x, p.x, (float)(r.K / 9 - 1) * Lx);
+					dy = exact_delta(O.y, p.y, (float)((r.K / 3) % 3 - 1) * Ly);
+					dz = exact_delta(O.z, p.z, (float)(r.K % 3 - 1) * Lz);
+				}
+				if (MODE == 0) {
+					tx = fmul(m4_w<COMP>(COMP ? sq3(dx, dy, dz) : d2, r.X.y, r.X.w), r.A.w);
+					if (dl) {
+						const float ih = __fsqrt_rn(r.X.y);      // 4 / fBall2 = 1 / h^2
+						ty = dlnk_term(sqrtf(sq3(dx, dy, dz)), ih, r.A.w) * (ih * ih * ih);
+					}
+				} else {
+					const float f = COMP ? grad_factor_f32(sq3(dx, dy, dz), r.X.y, r.X.z) : grad_factor(d2, r.X.y, r.X.z);
+					tx = fmul(dx, f); ty = fmul(dy, f); tz = fmul(dz, f);
+					if (ehit) ehit[r.e] = stamp;
+					else hmin = __builtin_amdgcn_fmed3f(r.X.w, -INFINITY, hmin);   // min; w is +inf for a density of 0
+				}
 			}
 		}
-		int nx = node;
-		while (nx & 1) nx >>= 1;
-		node = nx + 1;
-		if (node == 1) node = 0;
+		const unsigned long long m = __ballot(hit);
+		if (!m) return;
+		if (hit) {
+			const int t = (nq + __popcll(m & same & below)) * sp + j;
+			qx[t] = tx;
+			if (MODE == 1 || dl) qy[t] = ty;
+			if (MODE == 1) qz[t] = tz;
+		}
+		nq += __popcll(m & same);
+		if (__any(nq + 64 / sp > qcap)) drain();      // the next round may queue 64 / S' more
+	};
+	// the entities of the nl leaves whose nodes are in s_fr[wv][c], in order
+	auto scan = [&](int c, int nl) {
+		int *fs = s_fr[wv][c], *fe = s_fr[wv][c ^ 1];
+		wave_lds_sync();
+		for (int t = lane; t < nl; t += 64) {
+			const int2 rg = leaf_range(lstart, fs[t] - nLeaf2, B, ne);
+			fs[t] = rg.x; fe[t] = rg.y;
+		}
+		wave_lds_sync();
+		if (B <= 64) {
+			const int lpr = 64 / bp, q = lane / bp, off = lane & (bp - 1);
+			auto get = [&](int t0) {
+				const int t = t0 + q;
+				const int e = t < nl ? fs[t] + off : 0;
+				return fetch(e, t < nl && e < fe[t]);
+			};
+			Rec nx = get(0);
+			for (int t0 = 0; t0 < nl; t0 += lpr) {
+				const Rec cu = nx;
+				if (t0 + lpr < nl) nx = get(t0 + lpr);
+				take(cu);
+			}
+		} else {
+			for (int t = 0; t < nl; ++t)
+				for (int e0 = fs[t]; e0 < fe[t]; e0 += 64) take(fetch(e0 + lane, e0 + lane < fe[t]));
+		}
+		wave_lds_sync();
+	};
+	auto open = [&](int node) {
+		const float4 lo = nlo[node], hi = nhi[node];
+		return brange_has(hi.w, pb) && point_box_d2<false>(lo, hi, p.x, p.y, p.z, 0.f) < lo.w;
+	};
+	const int depth = __builtin_ctz(nLeaf2);
+	int lev = min(depth, 6), f, cur = 0;
+	bool over = false;
+	{
+		const bool ok = lane < (1 << lev) && open((1 << lev) + lane);
+		const unsigned long long m = __ballot(ok);
+		if (ok) s_fr[wv][0][__popcll(m & below)] = (1 << lev) + lane;
+		f = __popcll(m);
 	}
-	// fold the S partial sums of each point (xor partners stay within the group)
-#pragma unroll
-	for (int o = S / 2; o > 0; o >>= 1) {
+	while (lev < depth && f > 0 && !over) {
+		int d = 1;
+		while (d < depth - lev && (f << (d + 1)) <= 64) ++d;
+		const int tot = f << d;
+		const int *src = s_fr[wv][cur];
+		int *dst = s_fr[wv][cur ^ 1], nf = 0;
+		wave_lds_sync();
+		for (int t0 = 0; t0 < tot; t0 += 64) {
+			const int t = t0 + lane;
+			const int node = t < tot ? (src[t >> d] << d) + (t & ((1 << d) - 1)) : 0;
+			const bool ok = t < tot && open(node);
+			const unsigned long long m = __ballot(ok);
+			const int c = __popcll(m);
+			if (nf + c > WV_F) { over = true; break; }
+			if (ok) dst[nf + __popcll(m & below)] = node;
+			nf += c;
+		}
+		f = nf;
+		lev += d;
+		cur ^= 1;
+	}
+	if (!over) {
+		if (f > 0) scan(cur, f);
+	} else {
+		int node = 1, nl = 0;
+		wave_lds_sync();
+		while (node) {
+			node = uniform_int(node);
+			const bool ok = open(node);
+			if (ok && node < nLeaf2) { node = 2 * node; continue; }
+			if (ok) {
+				if (lane == 0) s_fr[wv][0][nl] = node;
+				if (++nl == WV_F) { scan(0, nl); nl = 0; }
+			}
+			node = (node >> __builtin_ctz(~node)) + 1;
+			if (node == 1) node = 0;
+		}
+		if (nl) scan(0, nl);
+	}
+	drain();
+	// fold the partial sums (every group of S' lanes holds the same ones)
+	for (int o = sp >> 1; o > 0; o >>= 1) {
 		s0.xor_merge(o);
 		if (MODE == 1 || dl) s1.xor_merge(o);
 		if (MODE == 1) s2.xor_merge(o);
 	}
-	if (MODE == 1 && bthr) box_min_atomic(hmin, valid, pb, bthr);
-	if (!valid || sub != 0) return;
+	if (MODE == 1 && bthr) box_min_atomic(hmin, true, pb, bthr);
+	if (lane != 0) return;
 	if (MODE == 0) {
 		out_sum[ii] = s0.val();
 		if (dl) out_dl[ii] = s1.val() * (float)(-M_1_PI / 6.0);
 		return;
 	}
-	const float fStep = micro ? bt[pb].fMicro : bt[pb].fStep;
-	const float ax = s0.val(), ay = s1.val(), az = s2.val();
-	const float ss = sq3(ax, ay, az);
-	float ai = (float)sqrt((double)ss);
-	if (ai > 0.0f) ai = (float)((double)fStep / sqrt((double)ss));
-	else ai = 0.0f;
-	float r[3] = {fsub(p.x, fmul(ai, ax)), fsub(p.y, fmul(ai, ay)), fsub(p.z, fmul(ai, az))};
-	const float C[3] = {cx, cy, cz}, LL[3] = {Lx, Ly, Lz};
-	for (int j = 0; j < 3; ++j) {
-		if ((double)r[j] > (double)C[j] + 0.5 * (double)LL[j]) r[j] = fsub(r[j], LL[j]);
-		if ((double)r[j] <= (double)C[j] - 0.5 * (double)LL[j]) r[j] = fadd(r[j], LL[j]);
-	}
-	ppos[pi] = make_float4(r[0], r[1], r[2], p.w);
+	move_point(ppos, pi, p, s0.val(), s1.val(), s2.val(), micro ? bt[pb].fMicro : bt[pb].fStep, cx, cy, cz, Lx, Ly,
+			Lz, nullptr);
 }
 
 // =====================================================================
@@ -2230,8 +2374,8 @@ static int cover_launch(skg_ctx *c, int mode, float4 *ppos, const int *plist, in
 			C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart, nullptr, nullptr, c->tlCap, nullptr, nullptr, 0, \
 			nullptr, out_dl, nullptr)
 #define CS(M_, C_)                                                                             \
-	k_cover_sub<M_, C_, 16><<<nblk(16L * np, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(ppos, plist, np, c->e_pos, \
-			c->e_aux, c->e_org, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, out, c->e_hit, stamp,       \
+	k_cover_wave<M_, C_, 16><<<nblk(64L * np, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(ppos, plist, np, c->e_pos, \
+			c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, out, c->e_hit, stamp,       \
 			nullptr, c->nBox > 1 ? pbox : nullptr, c->d_bt, micro, C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart, \
 			nullptr, nullptr, out_dl)
 	if (np <= c->subMax) {
@@ -2505,12 +2649,12 @@ static int enqueue_steps(skg_ctx *c, long cap, bool sub, bool lists, int nsteps,
 			k_bump<<<1, 1, 0, c->st>>>(c->d_ml);
 		const int pslot = capturing ? -1 : skg_prof_begin(c);
 #define MV(C_)                                                                                                \
-		if (sub && cap <= c->s64Max) k_cover_sub<1, C_, 64><<<nblk(64L * cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>( \
-				c->m_pos, c->m_list, (int)cap, c->e_pos, c->e_aux, c->e_org, c->nE, c->te.lo, c->te.hi,          \
+		if (sub && cap <= c->s64Max) k_cover_wave<1, C_, 64><<<nblk(64L * cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>( \
+				c->m_pos, c->m_list, (int)cap, c->e_pos, c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi,          \
 				c->te.nLeaf2, c->te.B, nullptr, ehit, 0, bthr, pbox, c->d_bt, micro, C[0], C[1], C[2], L[0],     \
 				L[1], L[2], c->te.lstart, c->d_ml + 1, c->d_ml, nullptr);                                        \
-		else if (sub) k_cover_sub<1, C_, 16><<<nblk(16L * cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos,  \
-				c->m_list, (int)cap, c->e_pos, c->e_aux, c->e_org, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2,      \
+		else if (sub) k_cover_wave<1, C_, 16><<<nblk(64L * cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, \
+				c->m_list, (int)cap, c->e_pos, c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2,      \
 				c->te.B, nullptr, ehit, 0, bthr, pbox, c->d_bt, micro, C[0], C[1], C[2], L[0], L[1],             \
 				L[2], c->te.lstart, c->d_ml + 1, c->d_ml, nullptr);                                              \
 		else k_cover<1, C_><<<nblk(cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_list, (int)cap,    \
