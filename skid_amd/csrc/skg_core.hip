@@ -449,33 +449,6 @@ __global__ void k_tree_level(float4 *lo, float4 *hi, int first, int count) {
 	hi[i] = make_float4(fmaxf(b0.x, b1.x), fmaxf(b0.y, b1.y), fmaxf(b0.z, b1.z), brange_pack(x0, x1));
 }
 
-// Refit of the entity tree's largest live ball alone: entities do not move and
-// ScatterCut only removes balls, so the position bounds stay as built and only
-// lo.w (the largest live fBall2 below; dead and filler entities carry -1)
-// changes.
-__global__ void k_leaf_ball(const float4 *__restrict__ eaux, int n, int B, int nLeaf, int nLeaf2,
-		const int *__restrict__ lstart, float4 *lo) {
-	const int l = blockIdx.x * blockDim.x + threadIdx.x;
-	if (l >= nLeaf2) return;
-	float w = -INFINITY;
-	if (l < nLeaf) {
-		const int2 r = leaf_range(lstart, l, B, n);
-		for (int i = r.x; i < r.y; ++i) w = fmaxf(w, eaux[i].x);
-	}
-	lo[nLeaf2 + l].w = w;
-}
-// The same for the leaves flagged by the sorted cut only (the others' entities
-// are unchanged since the last refit); clears the flags.
-__global__ void k_leaf_ball_dirty(const float4 *__restrict__ eaux, int n, int B, int nLeaf, int nLeaf2,
-		const int *__restrict__ lstart, float4 *lo, int *dirty) {
-	const int l = blockIdx.x * blockDim.x + threadIdx.x;
-	if (l >= nLeaf || !dirty[l]) return;
-	dirty[l] = 0;
-	float w = -INFINITY;
-	const int2 r = leaf_range(lstart, l, B, n);
-	for (int i = r.x; i < r.y; ++i) w = fmaxf(w, eaux[i].x);
-	lo[nLeaf2 + l].w = w;
-}
 // entity -> leaf, and no leaf flagged
 __global__ void k_entity_leaf(int n, int B, int nLeaf, int nLeaf2, const int *__restrict__ lstart, int *eleaf,
 		int *dirty) {
@@ -486,27 +459,48 @@ __global__ void k_entity_leaf(int n, int B, int nLeaf, int nLeaf2, const int *__
 	const int2 r = leaf_range(lstart, l, B, n);
 	for (int i = r.x; i < r.y; ++i) eleaf[i] = l;
 }
-__global__ void k_level_ball(float4 *lo, int first, int count) {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= count) return;
-	const int i = first + t;
-	lo[i].w = fmaxf(lo[2 * i].w, lo[2 * i + 1].w);
-}
-
-// The levels of at most mtop nodes in one workgroup, level by level (one
-// launch instead of one per level).  A level reads what the one below wrote
-// in the same launch: stores complete to L2 (agent fence) before the barrier,
-// and the reads bypass the CU's L1.
-__global__ __launch_bounds__(1024) void k_level_ball_top(float4 *lo, int mtop) {
-	for (int m = mtop; m >= 1; m >>= 1) {
-		for (int t = threadIdx.x; t < m; t += blockDim.x) {
-			const int i = m + t;
-			const float a = __hip_atomic_load(&lo[2 * i].w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			const float b = __hip_atomic_load(&lo[2 * i + 1].w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			lo[i].w = fmaxf(a, b);
+// Refit of the entity tree's largest live ball alone: entities do not move and
+// ScatterCut only removes balls, so the position bounds stay as built and only
+// lo.w (the largest live fBall2 below; dead and filler entities carry -1)
+// changes.  One workgroup takes BALL_CH consecutive nodes of a level (nc nodes,
+// ids nc ...) and writes every node above them that they alone decide, level by
+// level in LDS: one launch per 10 levels instead of one per level (3.8 us for
+// 256 leaves; 35 us level by level through L2 in one workgroup).  LEAF: the
+// nodes are leaves, recomputed first -- all of them, or with dirty only those
+// the sorted cut flagged (their flags are cleared).
+#define BALL_CH 1024
+template <bool LEAF>
+__global__ __launch_bounds__(256) void k_ball_up(const float4 *__restrict__ eaux, int n, int B, int nLeaf,
+		const int *__restrict__ lstart, float4 *lo, int nc, int *dirty) {
+	__shared__ float sv[BALL_CH];
+	const int cw = min(nc, BALL_CH), c0 = blockIdx.x * cw, tid = threadIdx.x;
+	for (int t = tid; t < cw; t += 256) {
+		const int l = c0 + t;
+		float w;
+		if (LEAF && (!dirty || (l < nLeaf && dirty[l]))) {
+			if (dirty) dirty[l] = 0;
+			w = -INFINITY;
+			if (l < nLeaf) {
+				const int2 r = leaf_range(lstart, l, B, n);
+				for (int i = r.x; i < r.y; ++i) w = fmaxf(w, eaux[i].x);
+			}
+			lo[nc + l].w = w;
+		} else {
+			w = lo[nc + l].w;
 		}
-		__threadfence();
+		sv[t] = w;
+	}
+	for (int m = cw >> 1, first = (nc + c0) >> 1; m >= 1; m >>= 1, first >>= 1) {
+		float v[2];
 		__syncthreads();
+#pragma unroll
+		for (int u = 0; u < 2; ++u) {
+			const int t = tid + 256 * u;
+			if (t < m) { v[u] = fmaxf(sv[2 * t], sv[2 * t + 1]); lo[first + t].w = v[u]; }
+		}
+		__syncthreads();
+#pragma unroll
+		for (int u = 0; u < 2; ++u) if (tid + 256 * u < m) sv[tid + 256 * u] = v[u];
 	}
 }
 
@@ -878,6 +872,9 @@ __global__ __launch_bounds__(64 * W) void k_knn(
 // reference's smx->pp).  MODE 0 accumulates the scatter half of the density,
 // MODE 1 the density gradient and then moves the point (kdMoveParticles).
 // =====================================================================
+// Whether a record whose w is w (the density, +inf for 0) is cut at threshold t.
+__device__ __forceinline__ bool cut_by(float w, float t) { return t > 0.f && (w < t || w == INFINITY); }
+
 // One entity e (record A, X, image code K) against the lane's point when want.
 // MODE 0 accumulates the scatter density (with dl also the scatter half of
 // d rho / d ln nSmooth into s1, exact separations, the factor -1/(6 pi)
@@ -888,10 +885,11 @@ __global__ __launch_bounds__(64 * W) void k_knn(
 template <int MODE, bool COMP, bool LAZYK = false>
 __device__ __forceinline__ void cover_hit(int e, const float4 &A, const float4 &X, int K, bool want,
 		const float4 &p, const float4 *__restrict__ eorg, int *__restrict__ ehit, int stamp, float &hmin,
-		float Lx, float Ly, float Lz, Sum<COMP> &s0, Sum<COMP> &s1, Sum<COMP> &s2, bool dl = false) {
+		float Lx, float Ly, float Lz, Sum<COMP> &s0, Sum<COMP> &s1, Sum<COMP> &s2, bool dl = false,
+		float cut = 0.f) {
 	float dx = fsub(A.x, p.x), dy = fsub(A.y, p.y), dz = fsub(A.z, p.z);
 	float d2 = sq3(dx, dy, dz);
-	if (want && d2 < X.x) {
+	if (want && d2 < X.x && !(MODE == 1 && cut_by(X.w, cut))) {
 		if (COMP || (MODE == 0 && dl)) {
 			// replica: separation from the source position plus the exact shift;
 			// LAZYK: the caller passes K < 0 and the code is read here, from the
@@ -930,7 +928,7 @@ __device__ __forceinline__ void cover_scan_staged(int start, int cnt, bool want,
 		const float4 *__restrict__ epos, const float4 *__restrict__ eaux, const float4 *__restrict__ eorg,
 		const int *__restrict__ ecode, int *__restrict__ ehit, int stamp, float &hmin, float Lx, float Ly,
 		float Lz, Sum<COMP> &s0, Sum<COMP> &s1, Sum<COMP> &s2, bool dl, float4 *sA, float4 *sX, int *sK,
-		int lane) {
+		int lane, float cut = 0.f) {
 	for (int c0 = 0; c0 < cnt; c0 += 64) {
 		const int m = min(64, cnt - c0);
 		if (lane < m) {
@@ -944,7 +942,7 @@ __device__ __forceinline__ void cover_scan_staged(int start, int cnt, bool want,
 		if (want)
 			for (int t = 0; t < m; ++t)
 				cover_hit<MODE, COMP>(start + c0 + t, sA[t], sX[t], sK[t], true, p, eorg, ehit, stamp, hmin, Lx, Ly,
-						Lz, s0, s1, s2, dl);
+						Lz, s0, s1, s2, dl, cut);
 		// every lane has read these records before the next chunk overwrites them
 		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 		__builtin_amdgcn_wave_barrier();
@@ -961,6 +959,7 @@ __device__ __forceinline__ void cover_scan_staged(int start, int cnt, bool want,
 // one address (device-scope atomics from every XCD serialise there);
 // k_thr_fold takes the minimum over the slots.  All 64 lanes must be active.
 #define SKG_THR_SLOTS 64
+#define SKG_BLOCK_STEPS 5     // PRUNE_STEPS: steps between prunes, a set of slots each
 __device__ __forceinline__ void box_min_atomic(float hmin, bool valid, int pb, int *bthr) {
 	const int lane = threadIdx.x & 63;
 	const bool has = valid && hmin < INFINITY;
@@ -976,6 +975,32 @@ __device__ __forceinline__ void box_min_atomic(float hmin, bool valid, int pb, i
 	}
 }
 
+// The box's ScatterCut threshold after the np steps before this one (their
+// slots, one set of nBox boxes per step): the largest of the steps' minima, 0
+// while no step has hit anything.  It never falls, so entities cut before the
+// run are below it too.  Every lane of the wavefront takes part; lanes of
+// several boxes are served box by box.
+__device__ __forceinline__ float cut_level(const float *__restrict__ slots, int nBox, int np, int pb) {
+	float t = 0.f;
+	if (np <= 0) return t;
+	const int lane = threadIdx.x & 63;
+	unsigned long long todo = ~0ull;
+	while (todo) {
+		const int b = __builtin_amdgcn_readlane(pb, __builtin_ctzll(todo));
+		float tb = 0.f, v[SKG_BLOCK_STEPS - 1];
+#pragma unroll
+		for (int s = 0; s < SKG_BLOCK_STEPS - 1; ++s)
+			v[s] = s < np ? slots[((size_t)s * nBox + b) * SKG_THR_SLOTS + lane] : INFINITY;
+#pragma unroll
+		for (int s = 0; s < SKG_BLOCK_STEPS - 1; ++s) {
+			const float m = wave_min(v[s]);
+			if (m < INFINITY) tb = fmaxf(tb, m);
+		}
+		if (pb == b) t = tb;
+		todo &= ~__ballot(pb == b);
+	}
+	return t;
+}
 // kdMoveParticles (kd.c:702-732) for one lane: a step of fStep against the
 // gradient (ax, ay, az), then the periodic wrap into the box; a wrap sets the
 // mover's flag (mwrap) that sends its wavefront back to the tree walk for the
@@ -1116,7 +1141,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		float cx, float cy, float cz, float Lx, float Ly, float Lz, const int *__restrict__ lstart,
 		const int *__restrict__ tlist, const int *__restrict__ tcnt, int tcap, const int *__restrict__ npDev,
 		const int *__restrict__ stampDev, int elist, const int *__restrict__ eblk, float *__restrict__ out_dl,
-		int *__restrict__ mwrap) {
+		int *__restrict__ mwrap, const float *__restrict__ cutSlots, int nBox, int nCut) {
 	if (npDev) np = *npDev;                       // device-resident active count and step stamp
 	if (stampDev) stamp = *stampDev;
 	// staging slots for the entity-list scan, 64 per wavefront
@@ -1134,6 +1159,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 	s0.init(); s1.init(); s2.init();
 	float hmin = INFINITY;
 	const bool dl = MODE == 0 && out_dl != nullptr;
+	const float cut = MODE == 1 ? cut_level(cutSlots, nBox, nCut, pb) : 0.f;
 	// With a leaf list for this tile (built at the start of the block, see
 	// k_cover_lists) the wavefront scans those leaves and walks no tree.
 	// Otherwise a node is opened when its largest live ball reaches at least
@@ -1187,7 +1213,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 						const int e = E2[u];
 						const bool mine = decltype(straddle)::value ? (valid && e >= elo && e < ehi) : valid;
 						cover_hit<MODE, COMP>(e, A2[u], X2[u], K2[u], mine, p, eorg, ehit, stamp, hmin, Lx, Ly, Lz,
-								s0, s1, s2);
+								s0, s1, s2, false, cut);
 					}
 				}
 				// every lane has read this chunk before the next overwrites it
@@ -1212,7 +1238,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		const int2 rg = leaf_range(lstart, leaf, B, ne);
 		cover_scan_staged<MODE, COMP>(uniform_int(rg.x), uniform_int(rg.y - rg.x), want, p, epos, eaux, eorg, ecode,
 				ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x & ~63), s_eX + (threadIdx.x & ~63),
-				s_eK + (threadIdx.x & ~63), lane);
+				s_eK + (threadIdx.x & ~63), lane, cut);
 	}
 	while (node) {
 		node = uniform_int(node);
@@ -1224,7 +1250,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 			const int2 rg = leaf_range(lstart, node - nLeaf2, B, ne);
 			cover_scan_staged<MODE, COMP>(uniform_int(rg.x), uniform_int(rg.y - rg.x), need, p, epos, eaux, eorg,
 					ecode, ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x & ~63),
-					s_eX + (threadIdx.x & ~63), s_eK + (threadIdx.x & ~63), lane);
+					s_eX + (threadIdx.x & ~63), s_eK + (threadIdx.x & ~63), lane, cut);
 		}
 		// next node in pre-order after node's subtree (strip trailing ones, step)
 		node = (node >> __builtin_ctz(~node)) + 1;
@@ -1415,7 +1441,8 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_cover_wave(
 		int nLeaf2, int B, float *__restrict__ out_sum, int *__restrict__ ehit, int stamp, int *__restrict__ bthr,
 		const int *__restrict__ pbox, const DevBox *__restrict__ bt, int micro,
 		float cx, float cy, float cz, float Lx, float Ly, float Lz, const int *__restrict__ lstart,
-		const int *__restrict__ npDev, const int *__restrict__ stampDev, float *__restrict__ out_dl) {
+		const int *__restrict__ npDev, const int *__restrict__ stampDev, float *__restrict__ out_dl,
+		const float *__restrict__ cutSlots, int nBox, int nCut) {
 	constexpr int NW = SKG_TILE_T / 64;
 	__shared__ int s_fr[NW][2][WV_F];
 	__shared__ float s_q[NW][3][WV_Q];
@@ -1428,6 +1455,7 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_cover_wave(
 	const float4 p = ppos[pi];
 	const int pb = pbox ? pbox[pi] : 0;
 	const bool dl = MODE == 0 && out_dl != nullptr;
+	const float cut = MODE == 1 ? cut_level(cutSlots, nBox, nCut, pb) : 0.f;
 	const unsigned long long below = (1ull << lane) - 1ull;
 	float *qx = s_q[wv][0], *qy = s_q[wv][1], *qz = s_q[wv][2];
 	// slots per leaf in a round of 64 lanes, and the lane j of the summation order
@@ -1468,7 +1496,7 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_cover_wave(
 		if (r.in) {
 			float dx = fsub(r.A.x, p.x), dy = fsub(r.A.y, p.y), dz = fsub(r.A.z, p.z);
 			const float d2 = sq3(dx, dy, dz);
-			if (d2 < r.X.x) {
+			if (d2 < r.X.x && !(MODE == 1 && cut_by(r.X.w, cut))) {
 				hit = true;
 				if ((COMP || dl) && r.K != 13) {  // 9(ix+1) + 3(iy+1) + (iz+1)
 					const float4 O = eorg[r.e];
@@ -1925,36 +1953,56 @@ __global__ void k_cut_bounds(const unsigned long long *__restrict__ key, int ne,
 		if (i < nBox) pos[i] = a;
 	}
 }
-__global__ __launch_bounds__(256) void k_cut_sorted(float *thr, const int *__restrict__ off,
+//
+// With slots it ends a run of nsteps steps at once (the move kernels skip what
+// the earlier steps' thresholds cut, see cut_level): the box's threshold after
+// step i is the largest of the steps' minima so far, log (optional) receives
+// the live count after each step, and the box's slots are reset for the next
+// run.  Without, thr holds the box's threshold of the step that just ran.  The
+// search narrows the range 256-fold a round (one dependent read each).
+__global__ __launch_bounds__(256) void k_cut_sorted(const float *__restrict__ thr, const int *__restrict__ off,
 		int *pos, const float *__restrict__ srho, const int *__restrict__ perm, int *elive, float4 *eaux,
-		int *bscat, int *liveTotal, const int *__restrict__ eleaf, int *dirty, const float *__restrict__ slots) {
-	__shared__ int snew;
-	const int b = blockIdx.x;
+		int *bscat, int *liveTotal, const int *__restrict__ eleaf, int *dirty, float *slots, int nsteps, int *log) {
+	__shared__ float st[SKG_BLOCK_STEPS];
+	const int b = blockIdx.x, nBox = gridDim.x, tid = threadIdx.x;
 	const int lo = pos[b], hi = off[b + 1];
-	// slots (optional): the box's SKG_THR_SLOTS partial minima, folded here
-	// (k_thr_fold's work, one launch fewer per step)
-	float tf = 0.f;
-	if (slots && threadIdx.x < 64) tf = wave_min(slots[(size_t)b * SKG_THR_SLOTS + threadIdx.x]);
-	if (threadIdx.x == 0) {
-		if (slots) thr[b] = tf;
-		const float t0 = slots ? tf : thr[b];
-		const float t = (t0 == INFINITY) ? 0.f : t0;
-		int a = lo, z = hi;
-		while (a < z) { const int m = (a + z) >> 1; if (srho[m] >= t) z = m; else a = m + 1; }
-		snew = a;
+	if (slots) {
+		for (int s = tid >> 6; s < nsteps; s += 4) {
+			float *p = slots + ((size_t)s * nBox + b) * SKG_THR_SLOTS + (tid & 63);
+			const float v = wave_min(*p);
+			*p = INFINITY;
+			if ((tid & 63) == 0) st[s] = v;
+		}
+		__syncthreads();
 	}
-	__syncthreads();
-	const int nw = snew;
-	for (int i = lo + (int)threadIdx.x; i < nw; i += blockDim.x) {
+	int nw = lo;
+	float t = 0.f;
+	for (int s = 0; s < (slots ? nsteps : 1); ++s) {
+		const float ts = slots ? st[s] : thr[b];
+		t = fmaxf(t, ts == INFINITY ? 0.f : ts);
+		if (slots && !log && s + 1 < nsteps) continue;        // only the last step's position is wanted
+		int z = hi;
+		while (z > nw) {                                      // the first position with srho >= t
+			const int g = (z - nw + 255) >> 8, i = nw + tid * g;
+			const int c = __syncthreads_count(i < z && srho[i] < t);
+			if (c == 0) break;
+			z = min(z, nw + c * g);
+			nw += (c - 1) * g + 1;
+		}
+		if (log && tid == 0) atomicAdd(&log[s], hi - nw);
+	}
+	for (int i = lo + tid; i < nw; i += blockDim.x) {
 		const int e = perm[i];
 		elive[e] = 0;
 		eaux[e].x = -1.f;
 		dirty[eleaf[e]] = 1;
 	}
-	if (threadIdx.x == 0) {
+	if (tid == 0) {
 		pos[b] = nw;
 		bscat[b] = hi - nw;
-		atomicAdd(liveTotal, hi - nw);
+		// with slots the total of the last cut goes down; without, it was zeroed before this one
+		if (!slots) atomicAdd(liveTotal, hi - nw);
+		else if (nw > lo) atomicSub(liveTotal, nw - lo);
 	}
 }
 
@@ -1963,25 +2011,105 @@ __global__ __launch_bounds__(256) void k_cut_sorted(float *thr, const int *__res
 // these, so the block can be replayed as one graph with no host round trip.
 __global__ void k_ml_set(int *ml, int i, int v) { ml[i] = v; }
 __global__ void k_bump(int *ml) { ml[0] += 1; }
-__global__ void k_ml_copy(int *ml) { ml[1] = ml[2]; }
 
-// Stream compaction of the active list by the prune flags: per-256 counts, a
-// one-workgroup scan of the counts, then ballot prefixes within each block.
-// Order is kept, so a Morton-sorted active list stays sorted.
-__global__ __launch_bounds__(256) void k_flag_counts(const int *__restrict__ flag, const int *__restrict__ nDev,
-		int *bcnt) {
+// kdPruneInactive test (kd.c:754-776): a mover stays active while it moved at
+// least fCvg over the last block; survivors restart from here.
+__device__ __forceinline__ bool prune_keep(const float4 *__restrict__ mpos, float4 *mold, int m, float hx, float hy,
+		float hz, float cv2) {
+	const float4 p = mpos[m], o = mold[m];
+	float dx = fsub(p.x, o.x), dy = fsub(p.y, o.y), dz = fsub(p.z, o.z);
+	if (dx > hx) dx = fsub(dx, 2 * hx);
+	if (dx <= -hx) dx = fadd(dx, 2 * hx);
+	if (dy > hy) dy = fsub(dy, 2 * hy);
+	if (dy <= -hy) dy = fadd(dy, 2 * hy);
+	if (dz > hz) dz = fsub(dz, 2 * hz);
+	if (dz <= -hz) dz = fadd(dz, 2 * hz);
+	const bool keep = sq3(dx, dy, dz) >= cv2;
+	if (keep) mold[m] = p;
+	return keep;
+}
+
+// The prune and the in-order compaction of the active list.  Small lists (at
+// most PRUNE_SMALL movers): one workgroup does all of it in one launch, up to
+// 16 consecutive movers a thread, their gathers in flight together; the list is
+// compacted in place (every thread has read its movers before the scan's
+// barriers, and survivors only move towards the front): 4.6 us against eight
+// launches of 4 us each; past 16 movers a thread the one workgroup becomes the
+// longer way.  bact: survivors per
+// box (the list is ordered by box).  ml[1] and ml[2] receive the count, and pin
+// (page-locked host memory) what the host waits for: pin[1] the count, pin[4]
+// the live-entity total.
+#define PRUNE_SMALL 16384
+__global__ __launch_bounds__(1024) void k_prune_small(int *list, int *ml, const float4 *__restrict__ mpos,
+		float4 *mold, float hx, float hy, float hz, const int *__restrict__ mbox, const DevBox *__restrict__ bt,
+		int nBox, int *bact, const int *__restrict__ liveTotal, int *pin) {
+	__shared__ int sw[16];
+	const int n = ml[1], tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+	const int per = (n + 1023) >> 10, i0 = tid * per;
+	int m[16], b[16];
+	unsigned keep = 0;
+#pragma unroll
+	for (int u = 0; u < 16; ++u) m[u] = u < per && i0 + u < n ? list[i0 + u] : -1;
+#pragma unroll
+	for (int u = 0; u < 16; ++u) b[u] = m[u] >= 0 ? mbox[m[u]] : 0;
+#pragma unroll
+	for (int u = 0; u < 16; ++u)
+		if (m[u] >= 0 && prune_keep(mpos, mold, m[u], hx, hy, hz, bt[b[u]].cvg2)) keep |= 1u << u;
+	for (int i = tid; i < nBox; i += 1024) bact[i] = 0;
+	const int c = __popc(keep);
+	int inc = c;
+#pragma unroll
+	for (int o = 1; o < 64; o <<= 1) {
+		const int v = __shfl_up(inc, o, 64);
+		if (lane >= o) inc += v;
+	}
+	if (lane == 63) sw[wv] = inc;
+	__syncthreads();
+	int off = inc - c, total = 0;
+#pragma unroll
+	for (int w = 0; w < 16; ++w) { if (w < wv) off += sw[w]; total += sw[w]; }
+	int run = 0;
+#pragma unroll
+	for (int u = 0; u < 16; ++u)
+		if (keep & (1u << u)) list[off++] = m[u];
+	if (nBox > 1) {
+		int rb = -1;
+#pragma unroll
+		for (int u = 0; u < 16; ++u)
+			if (keep & (1u << u)) {
+				if (b[u] != rb) { if (run) atomicAdd(&bact[rb], run); rb = b[u]; run = 0; }
+				++run;
+			}
+		if (run) atomicAdd(&bact[rb], run);
+	} else if (tid == 0) {
+		bact[0] = total;
+	}
+	if (tid == 0) { ml[1] = total; ml[2] = total; pin[1] = total; pin[4] = liveTotal[0]; }
+}
+
+// Larger lists: flags with per-256 counts, a one-workgroup scan of the counts,
+// ballot prefixes within each 256, then the copy back with the box counts.
+__global__ __launch_bounds__(256) void k_prune(const int *__restrict__ list, const int *__restrict__ naDev,
+		const float4 *__restrict__ mpos, float4 *mold, float hx, float hy, float hz, const int *__restrict__ mbox,
+		const DevBox *__restrict__ bt, int *flag, int *bcnt) {
 	__shared__ int sm[4];
-	const int n = *nDev;
-	const int i = blockIdx.x * 256 + threadIdx.x;
-	const int f = i < n ? flag[i] : 0;
+	const int n = *naDev, i = blockIdx.x * 256 + threadIdx.x;
+	int f = 0;
+	if (i < n) {
+		const int m = list[i];
+		f = prune_keep(mpos, mold, m, hx, hy, hz, bt[mbox[m]].cvg2);
+		flag[i] = f;
+	}
 	const int c = __popcll(__ballot(f));
 	if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = c;
 	__syncthreads();
 	if (threadIdx.x == 0) bcnt[blockIdx.x] = sm[0] + sm[1] + sm[2] + sm[3];
 }
-__global__ __launch_bounds__(1024) void k_scan_counts(const int *__restrict__ bcnt, int nb, int *boff, int *total) {
+__global__ __launch_bounds__(1024) void k_scan_counts(const int *__restrict__ bcnt, int nb, int *boff, int *total,
+		int *bact, int nBox) {
 	__shared__ int sm[1024];
 	const int t = threadIdx.x;
+	for (int i = t; i < nBox; i += 1024) bact[i] = 0;
 	const int per = (nb + 1023) / 1024;
 	const int a = min(nb, t * per), b = min(nb, a + per);
 	int sum = 0;
@@ -2012,52 +2140,13 @@ __global__ __launch_bounds__(256) void k_compact_dev(const int *__restrict__ lis
 	for (int k = 0; k < w; ++k) off += sm[k];
 	if (f) out[off + __popcll(m & ((1ull << lane) - 1ull))] = list[i];
 }
-__global__ void k_copy_list(const int *__restrict__ in, int *ml, int *out) {
-	const int n = ml[2];
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n) out[i] = in[i];
-}
 
-
-// kdPruneInactive test (kd.c:754-776): a mover stays active while it moved at
-// least fCvg over the last block; survivors restart from here.
-__global__ void k_prune(const int *__restrict__ list, const int *__restrict__ naDev, const float4 *__restrict__ mpos,
-		float4 *mold, float hx, float hy, float hz, const int *__restrict__ mbox, const DevBox *__restrict__ bt,
-		int *flag) {
-	const int na = *naDev;
-	int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= na) return;
-	int m = list[i];
-	const float cv2 = bt[mbox[m]].cvg2;
-	float4 p = mpos[m], o = mold[m];
-	float dx = fsub(p.x, o.x), dy = fsub(p.y, o.y), dz = fsub(p.z, o.z);
-	if (dx > hx) dx = fsub(dx, 2 * hx);
-	if (dx <= -hx) dx = fadd(dx, 2 * hx);
-	if (dy > hy) dy = fsub(dy, 2 * hy);
-	if (dy <= -hy) dy = fadd(dy, 2 * hy);
-	if (dz > hz) dz = fsub(dz, 2 * hz);
-	if (dz <= -hz) dz = fadd(dz, 2 * hz);
-	int keep = sq3(dx, dy, dz) >= cv2;
-	flag[i] = keep;
-	if (keep) mold[m] = p;
-}
-
-__global__ void k_compact(const int *__restrict__ list, const int *__restrict__ flag,
-		const int *__restrict__ off, int n, int *out) {
-	int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n && flag[i]) out[off[i]] = list ? list[i] : i;
-}
-
-// Active movers per box (lanes of one box add once per wavefront).
 // Active movers per box.  The active list is ordered by box (the movers are
 // sorted by box, then along the curve, and every prune compacts the list in
 // order), so the thread at a box's last mover finds the box's first by binary
 // search and writes the count; no atomics.  Boxes with no mover keep 0.
-__global__ void k_box_count(const int *__restrict__ list, const int *__restrict__ nDev, const int *__restrict__ mbox,
+__device__ __forceinline__ void box_count(const int *__restrict__ list, int n, const int *__restrict__ mbox, int i,
 		int *cnt) {
-	const int n = *nDev;
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n) return;
 	const int b = mbox[list[i]];
 	if (i + 1 < n && mbox[list[i + 1]] == b) return;
 	int lo = 0, hi = i;                            // the first index whose box is >= b
@@ -2067,6 +2156,25 @@ __global__ void k_box_count(const int *__restrict__ list, const int *__restrict_
 		else hi = m;
 	}
 	cnt[b] = i + 1 - lo;
+}
+__global__ void k_box_count(const int *__restrict__ list, const int *__restrict__ nDev, const int *__restrict__ mbox,
+		int *cnt) {
+	const int n = *nDev;
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n) box_count(list, n, mbox, i, cnt);
+}
+__global__ void k_copy_list(const int *__restrict__ in, int *ml, int *out, const int *__restrict__ mbox, int *bact,
+		const int *__restrict__ liveTotal, int *pin) {
+	const int n = ml[2];
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n) { out[i] = in[i]; box_count(in, n, mbox, i, bact); }
+	if (i == 0) { ml[1] = n; pin[1] = n; pin[4] = liveTotal[0]; }
+}
+
+__global__ void k_compact(const int *__restrict__ list, const int *__restrict__ flag,
+		const int *__restrict__ off, int n, int *out) {
+	int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n && flag[i]) out[off[i]] = list ? list[i] : i;
 }
 
 // CutCriterion (kd.c:555-597) per particle by iOrder.
@@ -2284,7 +2392,7 @@ extern "C" int skg_load_batch(skg_ctx *c, int nBox, const int *nGas, const int *
 	if (dalloc(&c->d_pos, 3 * n) || dalloc(&c->d_vel, 3 * n) || dalloc(&c->d_mass, n) ||
 	    dalloc(&c->d_soft, n) || dalloc(&c->d_temp, n) || dalloc(&c->d_rho, n) || dalloc(&c->d_ball2, n) ||
 	    dalloc(&c->d_grp, n) || dalloc(&c->d_boxOf, n) || dalloc(&c->d_type, n) || dalloc(&c->d_bt, nBox) ||
-	    dalloc(&c->d_bact, nBox) || dalloc(&c->d_bscat, nBox) || dalloc(&c->d_bthr, nBox) || dalloc(&c->d_bslot, (size_t)nBox * SKG_THR_SLOTS) ||
+	    dalloc(&c->d_bact, nBox) || dalloc(&c->d_bscat, nBox) || dalloc(&c->d_bthr, nBox) || dalloc(&c->d_bslot, (size_t)nBox * SKG_THR_SLOTS * SKG_BLOCK_STEPS) ||
 	    dalloc(&dbi, 3 * (size_t)nBox))
 		return SKG_E_NOMEM;
 	SKG_HIP(hipMemcpyAsync(c->d_bt, db.data(), sizeof(DevBox) * nBox, hipMemcpyHostToDevice, c->st));
@@ -2372,12 +2480,12 @@ static int cover_launch(skg_ctx *c, int mode, float4 *ppos, const int *plist, in
 	k_cover<M_, C_><<<nb, SKG_TILE_T, 0, c->st>>>(ppos, plist, np, c->e_pos, c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, \
 			c->te.hi, c->te.nLeaf2, c->te.B, out, c->e_hit, stamp, nullptr, c->nBox > 1 ? pbox : nullptr, c->d_bt, micro, \
 			C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart, nullptr, nullptr, c->tlCap, nullptr, nullptr, 0, \
-			nullptr, out_dl, nullptr)
+			nullptr, out_dl, nullptr, nullptr, 1, 0)
 #define CS(M_, C_)                                                                             \
 	k_cover_wave<M_, C_, 16><<<nblk(64L * np, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(ppos, plist, np, c->e_pos, \
 			c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, out, c->e_hit, stamp,       \
 			nullptr, c->nBox > 1 ? pbox : nullptr, c->d_bt, micro, C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart, \
-			nullptr, nullptr, out_dl)
+			nullptr, nullptr, out_dl, nullptr, 1, 0)
 	if (np <= c->subMax) {
 		if (mode == 0) { if (comp) CS(0, true); else CS(0, false); }
 		else { if (comp) CS(1, true); else CS(1, false); }
@@ -2634,34 +2742,41 @@ static int enqueue_steps(skg_ctx *c, long cap, bool sub, bool lists, int nsteps,
 	// can cross it in time for two or more of the block's list steps (closer
 	// to the margin the build walks more than the list steps save)
 	const float wsteps = 1.02f * (nsteps - 2);
+	// With the entities sorted by density, a step's cut is not applied before
+	// the next step: the move kernels skip what lies below the thresholds so
+	// far, and one k_cut_sorted ends the run.  With the one-launch prune and
+	// refit a block of five steps over a small list is 8 launches (31 before),
+	// a whole pass 10.7 -> 8.7 ms for 2,048 points and 19.4 -> 16.5 for 32,768.
+	const bool lazy = fusedThr && c->cutReady && !bInitial && nsteps <= SKG_BLOCK_STEPS;
 	if (lists && !fusedBuild) enqueue_lists(c, cap, nsteps, micro);
 	for (int i = 0; i < nsteps; ++i) {
 		// the initial step stamps its hits (unhit entities get density 0);
 		// later steps take the threshold from the move kernel itself
 		// (SKG_FUSED_THR=0: stamps and a pass over the entities every step)
 		const bool stamps = bInitial || !fusedThr;
+		const int nCut = lazy ? i : 0;
 		int *ehit = stamps ? c->e_hit : nullptr;
-		int *bthr = stamps ? nullptr : (int *)c->d_bslot;
-		if (!stamps)
+		int *bthr = stamps ? nullptr : (int *)c->d_bslot + (size_t)nCut * c->nBox * SKG_THR_SLOTS;
+		if (stamps)
+			k_bump<<<1, 1, 0, c->st>>>(c->d_ml);
+		else if (!lazy)
 			k_thr_reset<<<nblk((long)c->nBox * SKG_THR_SLOTS, 256), 256, 0, c->st>>>(c->d_bslot,
 					c->nBox * SKG_THR_SLOTS, c->d_cnt, c->d_ml);
-		else
-			k_bump<<<1, 1, 0, c->st>>>(c->d_ml);
 		const int pslot = capturing ? -1 : skg_prof_begin(c);
 #define MV(C_)                                                                                                \
 		if (sub && cap <= c->s64Max) k_cover_wave<1, C_, 64><<<nblk(64L * cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>( \
 				c->m_pos, c->m_list, (int)cap, c->e_pos, c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi,          \
 				c->te.nLeaf2, c->te.B, nullptr, ehit, 0, bthr, pbox, c->d_bt, micro, C[0], C[1], C[2], L[0],     \
-				L[1], L[2], c->te.lstart, c->d_ml + 1, c->d_ml, nullptr);                                        \
+				L[1], L[2], c->te.lstart, c->d_ml + 1, c->d_ml, nullptr, c->d_bslot, c->nBox, nCut);             \
 		else if (sub) k_cover_wave<1, C_, 16><<<nblk(64L * cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, \
 				c->m_list, (int)cap, c->e_pos, c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2,      \
 				c->te.B, nullptr, ehit, 0, bthr, pbox, c->d_bt, micro, C[0], C[1], C[2], L[0], L[1],             \
-				L[2], c->te.lstart, c->d_ml + 1, c->d_ml, nullptr);                                              \
+				L[2], c->te.lstart, c->d_ml + 1, c->d_ml, nullptr, c->d_bslot, c->nBox, nCut);                   \
 		else k_cover<1, C_><<<nblk(cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_list, (int)cap,    \
 				c->e_pos, c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, nullptr, \
 				ehit, 0, bthr, pbox, c->d_bt, micro, C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart,           \
 				lists ? c->tl_list : nullptr, lists ? c->tl_cnt : nullptr, c->tlCap, c->d_ml + 1, c->d_ml,  \
-				c->useLists != 2, c->d_eblk, nullptr, lists ? c->m_wrap : nullptr)
+				c->useLists != 2, c->d_eblk, nullptr, lists ? c->m_wrap : nullptr, c->d_bslot, c->nBox, nCut)
 #define MB(C_)                                                                                                \
 		k_cover_build<C_><<<nblk(cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_list, (int)cap, c->e_pos, \
 				c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, ehit, bthr, pbox,   \
@@ -2675,23 +2790,28 @@ static int enqueue_steps(skg_ctx *c, long cap, bool sub, bool lists, int nsteps,
 		if (pslot >= 0)
 			skg_prof_end(c, pslot, fusedBuild && i == 0 ? SKG_K_COVER_BUILD : SKG_K_COVER_MOVE,
 					24.0 * c->nActive + 24.0 * c->nLive);
+		if (lazy) continue;
 		if (stamps) {
 			k_scat_thr<<<nb, 256, 0, c->st>>>(c->e_live, c->e_hit, c->e_rho, c->e_aux, c->nE, c->d_ml, bInitial,
 					c->part);
 			k_box_min<<<c->nBox, 64, 0, c->st>>>(c->part, c->d_eblk, c->d_bthr, c->d_cnt);
-		} else if (!(c->cutReady && !bInitial)) {
+		} else {
 			k_thr_fold<<<c->nBox, SKG_THR_SLOTS, 0, c->st>>>(c->d_bslot, c->d_bthr);
 		}
 		if (c->cutReady && !bInitial) {
 			k_cut_sorted<<<c->nBox, 256, 0, c->st>>>(c->d_bthr, c->cs_off, c->cs_pos, c->cs_rho, c->cs_perm,
-					c->e_live, c->e_aux, c->d_bscat, c->d_cnt, c->e_leaf, c->leafDirty,
-					stamps ? nullptr : c->d_bslot);
+					c->e_live, c->e_aux, c->d_bscat, c->d_cnt, c->e_leaf, c->leafDirty, nullptr, 1, nullptr);
 		} else {
 			k_scat_cut<<<nb, 256, 0, c->st>>>(c->e_live, c->e_aux, c->e_rho, c->nE, c->e_box, c->d_bthr,
 					(int *)c->part);
 			k_box_sum<<<c->nBox, 64, 0, c->st>>>((const int *)c->part, c->d_eblk, c->d_bscat, c->d_cnt);
 		}
 		if (cntLog) k_log_count<<<1, 1, 0, c->st>>>(c->d_cnt, cntLog + i);
+	}
+	if (lazy) {
+		if (cntLog) k_fill_i<<<1, 64, 0, c->st>>>(cntLog, nsteps, 0);
+		k_cut_sorted<<<c->nBox, 256, 0, c->st>>>(nullptr, c->cs_off, c->cs_pos, c->cs_rho, c->cs_perm, c->e_live,
+				c->e_aux, c->d_bscat, c->d_cnt, c->e_leaf, c->leafDirty, c->d_bslot, nsteps, cntLog);
 	}
 	SKG_HIP(hipGetLastError());
 	return 0;
@@ -2705,38 +2825,40 @@ static int enqueue_prune(skg_ctx *c, long cap) {
 	const float *L = c->P.fPeriod;
 	const float hx = 0.5f * L[0], hy = 0.5f * L[1], hz = 0.5f * L[2];
 	const int nb = nblk(cap, 256);
-	k_prune<<<nb, 256, 0, c->st>>>(c->m_list, c->d_ml + 1, c->m_pos, c->m_old, hx, hy, hz, c->m_box, c->d_bt,
-			c->m_flag);
-	k_flag_counts<<<nb, 256, 0, c->st>>>(c->m_flag, c->d_ml + 1, c->m_bcnt);
-	k_scan_counts<<<1, 1024, 0, c->st>>>(c->m_bcnt, nb, c->m_bcnt + nb, c->d_ml + 2);
-	k_compact_dev<<<nb, 256, 0, c->st>>>(c->m_list, c->m_flag, c->d_ml + 1, c->m_bcnt + nb, c->m_list2);
-	k_copy_list<<<nb, 256, 0, c->st>>>(c->m_list2, c->d_ml, c->m_list);
-	k_ml_copy<<<1, 1, 0, c->st>>>(c->d_ml);
-	int rc;
-	if ((rc = count_active(c, cap))) return rc;
+	if (cap <= PRUNE_SMALL) {
+		k_prune_small<<<1, 1024, 0, c->st>>>(c->m_list, c->d_ml, c->m_pos, c->m_old, hx, hy, hz, c->m_box, c->d_bt,
+				c->nBox, c->d_bact, c->d_cnt, c->h_pin);
+	} else {
+		k_prune<<<nb, 256, 0, c->st>>>(c->m_list, c->d_ml + 1, c->m_pos, c->m_old, hx, hy, hz, c->m_box, c->d_bt,
+				c->m_flag, c->m_bcnt);
+		k_scan_counts<<<1, 1024, 0, c->st>>>(c->m_bcnt, nb, c->m_bcnt + nb, c->d_ml + 2, c->d_bact, c->nBox);
+		k_compact_dev<<<nb, 256, 0, c->st>>>(c->m_list, c->m_flag, c->d_ml + 1, c->m_bcnt + nb, c->m_list2);
+		k_copy_list<<<nb, 256, 0, c->st>>>(c->m_list2, c->d_ml, c->m_list, c->m_box, c->d_bact, c->d_cnt, c->h_pin);
+	}
 	return refit_entities(c);
 }
 
 static int refit_entities(skg_ctx *c) {
 	DevTree *t = &c->te;
 	// with the sorted cut every cut entity's leaf is flagged; before it, all
-	if (c->cutReady)
-		k_leaf_ball_dirty<<<nblk(t->nLeaf, 256), 256, 0, c->st>>>(c->e_aux, t->n, t->B, t->nLeaf, t->nLeaf2,
-				t->lstart, t->lo, c->leafDirty);
-	else
-		k_leaf_ball<<<nblk(t->nLeaf2, 256), 256, 0, c->st>>>(c->e_aux, t->n, t->B, t->nLeaf, t->nLeaf2, t->lstart,
-				t->lo);
-	int m = t->nLeaf2 >> 1;
-	for (; m > 2048; m >>= 1) k_level_ball<<<nblk(m, 256), 256, 0, c->st>>>(t->lo, m, m);
-	if (m >= 1) k_level_ball_top<<<1, 1024, 0, c->st>>>(t->lo, m);
+	int nc = t->nLeaf2;
+	k_ball_up<true><<<std::max(1, nc / BALL_CH), 256, 0, c->st>>>(c->e_aux, t->n, t->B, t->nLeaf, t->lstart, t->lo, nc,
+			c->cutReady ? c->leafDirty : nullptr);
+	while (nc > BALL_CH) {
+		nc /= BALL_CH;
+		k_ball_up<false><<<std::max(1, nc / BALL_CH), 256, 0, c->st>>>(nullptr, 0, 0, 0, nullptr, t->lo, nc, nullptr);
+	}
 	SKG_HIP(hipGetLastError());
 	return 0;
 }
 
-// Host copies of the live-entity total and the active count.
-static int read_counts(skg_ctx *c, int *nLive) {
-	SKG_HIP(hipMemcpyAsync(c->h_pin, c->d_ml, 12, hipMemcpyDeviceToHost, c->st));
-	SKG_HIP(hipMemcpyAsync(c->h_pin + 4, c->d_cnt, 4, hipMemcpyDeviceToHost, c->st));
+// Host copies of the live-entity total and the active count (pinned: the
+// prune's last kernel has written them to h_pin itself).
+static int read_counts(skg_ctx *c, int *nLive, bool pinned = false) {
+	if (!pinned) {
+		SKG_HIP(hipMemcpyAsync(c->h_pin, c->d_ml, 12, hipMemcpyDeviceToHost, c->st));
+		SKG_HIP(hipMemcpyAsync(c->h_pin + 4, c->d_cnt, 4, hipMemcpyDeviceToHost, c->st));
+	}
 	SKG_HIP(hipStreamSynchronize(c->st));
 	c->nActive = c->h_pin[1];
 	c->nLive = c->h_pin[4];
@@ -2829,6 +2951,9 @@ static int build_sorted_cut(skg_ctx *c) {
 	if ((rc = skg_sort_pairs(c, k0, k1, v0, v1, ne, 64))) return done(rc);
 	k_cut_bounds<<<nblk(std::max(ne, nBox + 1), 256), 256, 0, c->st>>>(k1, ne, nBox, c->cs_off, c->cs_pos,
 			c->cs_rho, v1, c->cs_perm);
+	// the steps' threshold slots start empty; each run's cut leaves them so
+	k_fill_f<<<nblk((long)nBox * SKG_THR_SLOTS * SKG_BLOCK_STEPS, 256), 256, 0, c->st>>>(c->d_bslot,
+			nBox * SKG_THR_SLOTS * SKG_BLOCK_STEPS, INFINITY);
 	hipError_t he = hipGetLastError();
 	if (he == hipSuccess) he = hipStreamSynchronize(c->st);
 	if (he != hipSuccess) { skg_note_hip(he, "build_sorted_cut", __FILE__, __LINE__); return done(SKG_E_HIP); }
@@ -2890,7 +3015,7 @@ extern "C" int skg_move_block(skg_ctx *c, int *nActive, int *nScatter) {
 		}
 		// nScatter of the Ittr line: the live count after the last step (the
 		// prune does not change it)
-		if ((rc = read_counts(c, &ns))) return rc;
+		if ((rc = read_counts(c, &ns, true))) return rc;
 		// Pruning thins the active list in its old order, so runs of 64 active
 		// movers spread out; once a tenth are gone, re-sort the rest by where
 		// they are now (per-mover sums do not depend on the order).  At most
