@@ -617,6 +617,11 @@ __global__ __launch_bounds__(COOP_T) void k_unb_coop(const int *__restrict__ bg,
 #define CAND_T 256
 #define CT 8
 #define CAND_WAVE 2048        // groups below this many members: one wavefront each
+// largest groups that k_unb_res holds in one wavefront, 256 and 512 threads
+#define RES_A 512
+#define RES_B 2048
+#define RES_C 8192
+#define RES_CUS 256           // CUs of an MI355X
 __device__ __forceinline__ float kernel_max(int soft, float twoh) {
 	return soft == SKG_PLUMMER ? 2.0f / twoh : 2.8f / twoh;     // K(0): spline 1.4*2/twoh, Plummer 2/twoh
 }
@@ -662,6 +667,28 @@ __device__ __forceinline__ void wave_argmax_dpp(double &E, int &i) {
 	E = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(E), 63),
 			__builtin_amdgcn_readlane(__double2loint(E), 63));
 	i = __builtin_amdgcn_readlane(i, 63);
+}
+// The same with the energies alone through the DPP steps (three instructions a
+// step, not eleven); the index comes from the lanes that hold the maximum.
+template <int CTRL, int RMASK>
+__device__ __forceinline__ double dpp_max_step(double E) {
+	const int lo = __double2loint(E), hi = __double2hiint(E);
+	return fmax(E, __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, RMASK, 0xF, false),
+			__builtin_amdgcn_update_dpp(lo, lo, CTRL, RMASK, 0xF, false)));
+}
+__device__ __forceinline__ void wave_argmax_fast(double &E, int &i) {
+	double m = dpp_max_step<0xB1, 0xF>(E);
+	m = dpp_max_step<0x4E, 0xF>(m);
+	m = dpp_max_step<0x141, 0xF>(m);
+	m = dpp_max_step<0x140, 0xF>(m);
+	m = dpp_max_step<0x142, 0xA>(m);
+	m = dpp_max_step<0x143, 0xC>(m);
+	m = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(m), 63),
+			__builtin_amdgcn_readlane(__double2loint(m), 63));
+	const unsigned long long eq = __ballot(E == m);
+	if (eq && !(eq & (eq - 1))) i = __builtin_amdgcn_readlane(i, __builtin_ctzll(eq));
+	else i = wave_min_i(E == m ? i : INT_MAX);        // a tie
+	E = m;
 }
 __device__ __forceinline__ double wave_max_d(double v) {
 #pragma unroll
@@ -939,6 +966,191 @@ __global__ __launch_bounds__(T) void k_unb_cand(const int *__restrict__ glist, c
 		atomicAdd(npairs, pairs);
 		atomicAdd(nfull, fulls);
 	}
+}
+
+// The same removal with every member resident, one workgroup per group of at
+// most T * SL members (member tid + c T in slot c of thread tid).  A full pass
+// of k_unb_cand over a group that dissolves buys only a removal or two (each
+// removal can raise a member's energy by K_max, far more than the gaps between
+// energies), so here a removal simply updates every member: with
+// u = fShift v + fCosmo r and phi (1+z) kept in FP64 registers it costs 8 FP64
+// and, with kdSubPot, some 14 FP32 operations a member and no memory traffic
+// (LQ: but one LDS read).  What is left is the chain [energies, argmax, barrier, the
+// winner's record, barrier, centre of mass] of each removal: 2.4 us in a group
+// of 1,643 members that dissolves, against 7 us in k_unb_cand with 84% of its
+// removals followed by a full pass (100,003 points: unbinding loops 19.5 ->
+// 4.0 ms; 50,021 points: 4.8 -> 2.1 ms).
+//
+// w = fShift vcm + fCosmo rcm is advanced by itself, w += f (w - u_b); vcm
+// and the mass for the catalogue follow the removals one behind, from memory,
+// so that their loads stay off the chain.
+template <int T, int SL, bool LQ>
+__global__ __launch_bounds__(T) void k_unb_res(const int *__restrict__ glist, const int *__restrict__ gs,
+		const int *__restrict__ ge, const float4 *__restrict__ uq, const float4 *__restrict__ uv,
+		const float2 *__restrict__ uphi, const int *__restrict__ uord, int *grp, int *gcount, float *gmass,
+		float4 *gvcm, float4 *grbound, const float4 *__restrict__ grel, float fShift, float fCosmo, float z, float G,
+		int soft, int bSub, int bNoUnbind, float hx, int *nunb, unsigned long long *npairs,
+		unsigned long long *nfull) {
+	constexpr int NW = T / 64;
+	__shared__ float4 sQ[LQ ? T * SL : 1];        // x, y, z, softening: every member's, or the removed one's
+	__shared__ double sA[NW], sU[4];
+	__shared__ int sI[NW];
+	const int g = glist[blockIdx.x], tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+	const int s = gs[g], n0 = ge[g] - s;
+	const double zf = 1.0 + (double)z;
+	auto sync = [&]() {
+		if (NW > 1) { __syncthreads(); return; }
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+	};
+	auto block_sum = [&](double v) {
+#pragma unroll
+		for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+		sync();
+		if (lane == 0) sA[wv] = v;
+		sync();
+		v = sA[0];
+#pragma unroll
+		for (int w = 1; w < NW; ++w) v += sA[w];
+		return v;
+	};
+	double U0[SL], U1[SL], U2[SL], P[SL];
+	float M[SL];
+	float4 Q[LQ ? 1 : SL];                        // position, softening (LQ: in sQ)
+	unsigned alive = 0, gone = 0;
+	double cm[7];
+	{
+		double a[7] = {0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+		for (int c = 0; c < SL; ++c) {
+			const int i = tid + c * T;
+			U0[c] = U1[c] = U2[c] = P[c] = 0.0;
+			M[c] = 0.f;
+			if (!LQ) Q[LQ ? 0 : c] = make_float4(0.f, 0.f, 0.f, 0.f);
+			if (i >= n0) continue;
+			const float4 q = uq[s + i], v = uv[s + i];
+			const float2 ph = uphi[s + i];
+			alive |= 1u << c;
+			(LQ ? sQ[i] : Q[LQ ? 0 : c]) = make_float4(q.x, q.y, q.z, v.w);
+			M[c] = q.w;
+			U0[c] = (double)fShift * (double)v.x + (double)fCosmo * (double)q.x;
+			U1[c] = (double)fShift * (double)v.y + (double)fCosmo * (double)q.y;
+			U2[c] = (double)fShift * (double)v.z + (double)fCosmo * (double)q.z;
+			P[c] = ((double)ph.x + (double)ph.y) * zf;
+			a[0] += (double)q.w;
+			a[1] += (double)fmul(q.w, q.x); a[2] += (double)fmul(q.w, q.y); a[3] += (double)fmul(q.w, q.z);
+			a[4] += (double)fmul(q.w, v.x); a[5] += (double)fmul(q.w, v.y); a[6] += (double)fmul(q.w, v.z);
+		}
+		for (int k = 0; k < 7; ++k) cm[k] = block_sum(a[k]);   // fp64 mass, centre and velocity (kd.c:1360-1375)
+		for (int k = 1; k < 7; ++k) cm[k] /= cm[0];
+	}
+	double w0 = (double)fShift * cm[4] + (double)fCosmo * cm[1];
+	double w1 = (double)fShift * cm[5] + (double)fCosmo * cm[2];
+	double w2 = (double)fShift * cm[6] + (double)fCosmo * cm[3];
+	double vc0 = cm[4], vc1 = cm[5], vc2 = cm[6], mass = cm[0];
+	double pf = 0.0;                              // the last removal, not yet in vcm
+	float4 pv = make_float4(0.f, 0.f, 0.f, 0.f);
+	const int vz = vgpr_zero();
+	auto energy = [&](int c) {
+		const double a = U0[c] - w0, b = U1[c] - w1, d = U2[c] - w2;
+		return fma(0.5, fma(a, a, fma(b, b, d * d)), -P[c]);
+	};
+	int n = n0, mi = INT_MAX;
+	unsigned long long pairs = 0;
+	while (!bNoUnbind && n > 0) {
+		double bE = -INFINITY;
+		int bi = INT_MAX;
+#pragma unroll
+		for (int c = 0; c < SL; ++c)
+			if (c * T < n0) {
+				const double E = energy(c);
+				if ((alive >> c & 1u) && E > bE) { bE = E; bi = tid + c * T; }
+			}
+		wave_argmax_fast(bE, bi);
+		if (NW > 1) {
+			if (lane == 0) { sA[wv] = bE; sI[wv] = bi; }
+			sync();
+			bE = sA[0]; bi = sI[0];
+#pragma unroll
+			for (int w = 1; w < NW; ++w) {
+				const double e = sA[w];
+				const int i = sI[w];
+				if (e > bE || (e == bE && i < bi)) { bE = e; bi = i; }
+			}
+		}
+		if (!(bE >= 0.0)) break;                  // every member is bound (kd.c:1412)
+		const int BI = uniform_int(bi), BC = BI / T, BT = BI % T;
+		if (wv == BT / 64) {
+#pragma unroll
+			for (int c = 0; c < SL; ++c)
+				if (c == BC && tid == BT) {
+					sU[0] = U0[c]; sU[1] = U1[c]; sU[2] = U2[c]; sU[3] = (double)M[c];
+					if (!LQ) sQ[0] = Q[LQ ? 0 : c];
+					alive &= ~(1u << c);
+					gone |= 1u << c;
+				}
+		}
+		sync();
+		const double mb = sU[3];
+		const float4 qb = sQ[LQ ? BI : 0];
+		if (wv == 0) {                            // the removal before this one: its record has arrived
+			vc0 += pf * (vc0 - (double)pv.x); vc1 += pf * (vc1 - (double)pv.y); vc2 += pf * (vc2 - (double)pv.z);
+			pv = uv[s + BI + vz];                 // a vector load: a scalar one would be waited for with the LDS reads
+		}
+		--n;
+		mass -= mb;
+		if (n == 0) { mi = BI; break; }
+		const double f = mb / mass;
+		pf = f;
+		w0 += f * (w0 - sU[0]); w1 += f * (w1 - sU[1]); w2 += f * (w2 - sU[2]);
+		if (bSub) {                               // kdSubPot (grav.c:39-60)
+			pairs += n;
+			const float gm = fmul(G, (float)mb);
+#pragma unroll
+			for (int c = 0; c < SL; ++c)
+				if (c * T < n0 && (alive >> c & 1u)) {
+					const float4 q = LQ ? sQ[tid + c * T] : Q[LQ ? 0 : c];
+					const float dx = fsub(qb.x, q.x), dy = fsub(qb.y, q.y), dz = fsub(qb.z, q.z);
+					P[c] -= zf * (double)fmul(gm, pot_kernel(soft, fmaf(dx, dx, fmaf(dy, dy, dz * dz)), fadd(qb.w, q.w)));
+				}
+		}
+		// (the next round's first barrier keeps its sU writes off these reads)
+	}
+	vc0 += pf * (vc0 - (double)pv.x); vc1 += pf * (vc1 - (double)pv.y); vc2 += pf * (vc2 - (double)pv.z);
+	if (n == 0) { mass = 0.0; vc0 = vc1 = vc2 = 0.0; }
+#pragma unroll
+	for (int c = 0; c < SL; ++c)
+		if (gone >> c & 1u) grp[uord[s + tid + c * T]] = 0;
+	// the most bound member left (kd.c:1400-1408 of the last pass; with none left
+	// the one that went last)
+	double mE = INFINITY;
+#pragma unroll
+	for (int c = 0; c < SL; ++c)
+		if (c * T < n0 && (alive >> c & 1u)) {
+			const double E = energy(c);
+			if (E < mE) { mE = E; mi = tid + c * T; }
+		}
+	wave_argmin_d(mE, mi);
+	sync();
+	if (lane == 0) { sA[wv] = mE; sI[wv] = mi; }
+	sync();
+	if (tid != 0) return;
+	for (int w = 1; w < NW; ++w)
+		if (sA[w] < mE || (sA[w] == mE && sI[w] < mi)) { mE = sA[w]; mi = sI[w]; }
+	gcount[g] = n;
+	gmass[g] = (float)mass;
+	gvcm[g] = make_float4((float)vc0, (float)vc1, (float)vc2, 0.f);
+	const float4 q = uq[s + (mi < n0 ? mi : 0)], r = grel[g];
+	float b[3] = {fadd(q.x, r.x), fadd(q.y, r.y), fadd(q.z, r.z)};
+	for (int j = 0; j < 3; ++j) {
+		if (b[j] > hx) b[j] = fsub(b[j], 2 * hx);
+		if (b[j] <= -hx) b[j] = fadd(b[j], 2 * hx);
+	}
+	grbound[g] = make_float4(b[0], b[1], b[2], 0.f);
+	atomicAdd(nunb, n0 - n);
+	atomicAdd(npairs, pairs);
+	atomicAdd(nfull, 1ull);
 }
 
 // Large groups, all at once in one cooperative launch, with the bounded
@@ -1612,11 +1824,28 @@ extern "C" int skg_unbind(skg_ctx *c, int *nUnbound) {
 		gmed.insert(gmed.end(), gbig.begin() + 128, gbig.end());
 		gbig.resize(128);
 	}
-	// groups below CAND_WAVE members run one wavefront each (512 candidates,
-	// no workgroup barriers), the rest 256 threads (2048 candidates); the
-	// small ones first in the list
-	const int nMedW = (int)(std::stable_partition(gmed.begin(), gmed.end(),
-			[&](int g) { return he[g] - hs[g] < CAND_WAVE; }) - gmed.begin());
+	// the list in order of the kernels.  With kdSubPot the groups whose members
+	// all stay resident run so, in one wavefront (up to RES_A members), 256
+	// (RES_B) or 512 threads (RES_C).  Without it the candidates' bound
+	// stays tight and k_unb_cand, which evaluates only those, is the faster past
+	// one wavefront's residents (a 2^21 gas+dark box: 20 ms against 32): one
+	// wavefront below CAND_WAVE members, 256 threads from there.
+	std::vector<int> nIn;
+	{
+		auto at = gmed.begin();
+		const int most[] = {RES_A, bSub0 ? RES_B : CAND_WAVE - 1, bSub0 ? RES_C : 0, INT_MAX};
+		for (int m : most) {
+			const auto to = std::stable_partition(at, gmed.end(), [&](int g) { return he[g] - hs[g] <= m; });
+			// the largest first: the last ones to start are then the shortest
+			if (m > RES_A) std::stable_sort(at, to, [&](int a, int b) { return he[a] - hs[a] > he[b] - hs[b]; });
+			nIn.push_back((int)(to - at));
+			at = to;
+		}
+		// a group of the third class takes a CU's LDS to itself: with more of
+		// them than CUs the candidates' smaller workgroups get through sooner
+		// (332 groups: 5.4 ms against 6.4)
+		if (nIn[2] > RES_CUS) { nIn[3] += nIn[2]; nIn[2] = 0; }
+	}
 	SKG_HIP(hipMemsetAsync(G->d_nunb, 0, 4, c->st));
 	const bool any = !gsmall.empty() || !gmed.empty() || !gbig.empty();
 	if (any) {
@@ -1696,28 +1925,28 @@ extern "C" int skg_unbind(skg_ctx *c, int *nUnbound) {
 		skg_prof_end(c, pslot, SKG_K_UNB_POT, 20.0 * pairs);
 		const int bSub = (c->inType == SKG_DARK || c->inType == SKG_STAR);   // kd.c:1441
 		const int lslot = skg_prof_begin(c);
-		// the sizes run side by side: groups of at most 64 members and the
-		// wavefront-sized ones on the context's second stream, forked from and
-		// joined back to the main one, the 256-thread groups on the main one
+		// the sizes run side by side: the larger ones on the main stream, the
+		// others on the context's second one, forked from and joined back to it
 		// (the groups are disjoint; the counters are atomic)
-		const bool fork = (nMedW > 0 || !gsmall.empty()) && (int)gmed.size() > nMedW;
+		const bool fork = (nIn[0] > 0 || nIn[1] > 0 || !gsmall.empty()) && (nIn[2] > 0 || nIn[3] > 0);
+		const hipStream_t s2 = fork ? c->st2 : c->st;
 		if (fork) {
 			SKG_HIP(hipEventRecord(c->evFork, c->st));
 			SKG_HIP(hipStreamWaitEvent(c->st2, c->evFork, 0));
 		}
-		if ((int)gmed.size() > nMedW)
-			k_unb_cand<CAND_T><<<(int)gmed.size() - nMedW, CAND_T, 0, c->st>>>(dgm + nMedW, G->gstart, G->gend,
-					G->uq, G->uv, G->uphi, G->uord, c->d_grp, G->count, G->mass, G->vcm, G->rbound, G->rel,
-					c->P.fShift, c->P.fCosmo, c->P.z, c->P.G, c->P.iSoftType, bSub, c->P.bNoUnbind, hx, G->d_nunb,
-					npair, npair + 2);
-		if (!gsmall.empty())
-			k_unb_small<<<(int)gsmall.size(), 64, 0, fork ? c->st2 : c->st>>>(dgs, G->gstart, G->gend, G->uq, G->uv,
-					G->uphi, G->uord, c->d_grp, G->count, G->mass, G->vcm, G->rbound, G->rel, c->P.fShift,
-					c->P.fCosmo, c->P.z, c->P.G, c->P.iSoftType, bSub, c->P.bNoUnbind, hx, G->d_nunb, npair);
-		if (nMedW > 0)
-			k_unb_cand<64><<<nMedW, 64, 0, fork ? c->st2 : c->st>>>(dgm, G->gstart, G->gend, G->uq, G->uv, G->uphi,
-					G->uord, c->d_grp, G->count, G->mass, G->vcm, G->rbound, G->rel, c->P.fShift, c->P.fCosmo, c->P.z,
-					c->P.G, c->P.iSoftType, bSub, c->P.bNoUnbind, hx, G->d_nunb, npair, npair + 2);
+#define SKG_UNB_ARGS(L_) L_, G->gstart, G->gend, G->uq, G->uv, G->uphi, G->uord, c->d_grp, G->count, G->mass, G->vcm, \
+			G->rbound, G->rel, c->P.fShift, c->P.fCosmo, c->P.z, c->P.G, c->P.iSoftType, bSub, c->P.bNoUnbind, hx,    \
+			G->d_nunb, npair
+		const int *l1 = dgm + nIn[0], *l2 = l1 + nIn[1], *l3 = l2 + nIn[2];
+		if (nIn[3] > 0) k_unb_cand<CAND_T><<<nIn[3], CAND_T, 0, c->st>>>(SKG_UNB_ARGS(l3), npair + 2);
+		if (nIn[2] > 0) k_unb_res<512, RES_C / 512, true><<<nIn[2], 512, 0, c->st>>>(SKG_UNB_ARGS(l2), npair + 2);
+		if (nIn[1] > 0) {
+			if (bSub) k_unb_res<256, RES_B / 256, false><<<nIn[1], 256, 0, s2>>>(SKG_UNB_ARGS(l1), npair + 2);
+			else k_unb_cand<64><<<nIn[1], 64, 0, s2>>>(SKG_UNB_ARGS(l1), npair + 2);
+		}
+		if (nIn[0] > 0) k_unb_res<64, RES_A / 64, false><<<nIn[0], 64, 0, s2>>>(SKG_UNB_ARGS(dgm), npair + 2);
+		if (!gsmall.empty()) k_unb_small<<<(int)gsmall.size(), 64, 0, s2>>>(SKG_UNB_ARGS(dgs));
+#undef SKG_UNB_ARGS
 		if (fork) {
 			SKG_HIP(hipEventRecord(c->evJoin, c->st2));
 			SKG_HIP(hipStreamWaitEvent(c->st, c->evJoin, 0));
