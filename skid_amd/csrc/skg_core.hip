@@ -872,6 +872,55 @@ __global__ __launch_bounds__(64 * W) void k_knn(
 // reference's smx->pp).  MODE 0 accumulates the scatter half of the density,
 // MODE 1 the density gradient and then moves the point (kdMoveParticles).
 // =====================================================================
+// ---- windows: which of up to 64 staged records a lane needs, as a bit mask.
+// A ball (or reach) of squared radius R around e holds the point p when
+//   e.p + (R - |e|^2)/2 > |p|^2/2
+// in coordinates relative to the tile's centre: three fma and a compare per
+// record and lane instead of nine operations and a branch, the compare's carry
+// shifted into the mask (the first record in the highest bit).  Rounding can
+// err by under 12 2^-24 (|e|^2 + |p|^2 + R); the bounds are widened by 4e-6 of
+// it (and an unordered compare passes), so the mask holds every record that the
+// exact test (cover_hit's) accepts; the few others are dropped there.
+__device__ __forceinline__ float4 win_record(const float4 &A, float R, const float4 &o) {
+	const float x = A.x - o.x, y = A.y - o.y, z = A.z - o.z, e2 = fmaf(x, x, fmaf(y, y, z * z));
+	return make_float4(x, y, z, R < 0.f ? -INFINITY : fmaf(4e-6f, e2 + R, 0.5f * (R - e2)));
+}
+__device__ __forceinline__ float4 win_point(const float4 &p, const float4 &o) {
+	const float x = p.x - o.x, y = p.y - o.y, z = p.z - o.z, p2 = fmaf(x, x, fmaf(y, y, z * z));
+	return make_float4(x, y, z, (0.5f - 4e-6f) * p2);
+}
+__device__ __forceinline__ void win_push(unsigned &m, const float4 &T, const float4 &w) {
+	const float t = fmaf(T.x, w.x, fmaf(T.y, w.y, fmaf(T.z, w.z, T.w)));
+	// m = 2 m + !(t <= w.w)
+	asm("v_cmp_nle_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(t), "v"(w.w) : "vcc");
+}
+// The masks of the 64 records at sT (padded with -inf past the end); the second
+// half is left empty when there are at most 32.
+__device__ __forceinline__ void win_masks(const float4 *sT, int cnt, const float4 &w, unsigned &m0, unsigned &m1) {
+	m0 = m1 = 0;
+#pragma unroll 8
+	for (int t = 0; t < 32; ++t) win_push(m0, sT[t], w);
+	if (cnt > 32) {
+#pragma unroll 8
+		for (int t = 32; t < 64; ++t) win_push(m1, sT[t], w);
+	}
+}
+// The or of every lane's v, in every lane.
+__device__ __forceinline__ unsigned wave_or(unsigned v) {
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);      // quad_perm [1,0,3,2]
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);      // quad_perm [2,3,0,1]
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);     // row_half_mirror
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);     // row_mirror
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);    // row_bcast:15 into rows 1 and 3
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);    // row_bcast:31 into rows 2 and 3
+	return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ void wave_lds_sync() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Whether a record whose w is w (the density, +inf for 0) is cut at threshold t.
 __device__ __forceinline__ bool cut_by(float w, float t) { return t > 0.f && (w < t || w == INFINITY); }
 
@@ -1028,32 +1077,23 @@ __device__ __forceinline__ void move_point(float4 *__restrict__ ppos, int pi, co
 	}
 }
 
-// Leaf lists for a block of move steps.  Entities do not move and ScatterCut
-// only removes balls, so while the active list (and with it every tile of 64
-// movers) is unchanged, the leaves any step can need are those whose ball
-// reach, widened by the distance a mover can still travel (margin), holds a
-// lane's point now.  One walk per block then replaces one walk per step.  A
-// tile with more than cap entries gets count -1 and walks the tree.  Near a
-// periodic face the listed entities include the replicas there; a mover that
-// crosses the face during the block jumps to the far side, which this list
-// does not cover, so the move step flags it (mwrap, cleared here: no face
-// covered) and its wavefront walks the tree for the rest of the block.  The
-// fused build (k_cover_build) also lists the far side of a lane's one near
-// face.
-//
-// ELIST: the list holds entities instead of leaves -- every live entity whose
-// ball, widened by the margin, holds a lane's point now, in tree order (leaf
-// by leaf, entities in index order, as the walk meets them), so a lane's hits
-// and its sums keep the walk's order.  A lane tests only leaves of its own
-// box, so every listed entity is of some lane's box.
-template <bool ELIST>
-__global__ __launch_bounds__(SKG_TILE_T) void k_cover_lists(const float4 *__restrict__ ppos,
+// Lists for a block of move steps.  Entities do not move and ScatterCut only
+// removes balls, so while the active list (and with it every tile of 64 movers)
+// is unchanged, what any step can need lies within a ball's reach of a lane's
+// point now, the reach widened by the distance a mover can still travel
+// (margin).  One walk per block then replaces one walk per step.  A tile with
+// more than cap entries gets count -1 and walks the tree.  Near a periodic face
+// the lists include the replicas there; a mover that crosses the face during
+// the block jumps to the far side, which its list may not cover: the move step
+// then flags it (mwrap) and its wavefront walks the tree for the rest of the
+// block.
+
+// Leaf lists (SKG_TILE_LISTS=2): the leaves a lane's point can reach.
+__global__ __launch_bounds__(SKG_TILE_T) void k_leaf_lists(const float4 *__restrict__ ppos,
 		const int *__restrict__ plist, int np, const float4 *__restrict__ nlo, const float4 *__restrict__ nhi,
 		int nLeaf2, const int *__restrict__ pbox, const DevBox *__restrict__ bt, int micro, float msteps,
-		float mabs, int per, float cx, float cy, float cz, float Lx, float Ly, float Lz, int cap,
-		int *__restrict__ tlist, int *__restrict__ tcnt, const int *__restrict__ npDev,
-		const float4 *__restrict__ epos, const float4 *__restrict__ eaux, const int *__restrict__ lstart, int B,
-		int ne, int *__restrict__ mwrap) {
+		float mabs, int cap, int *__restrict__ tlist, int *__restrict__ tcnt, const int *__restrict__ npDev,
+		int *__restrict__ mwrap) {
 	if (npDev) np = *npDev;
 	const int lane = threadIdx.x & 63;
 	const int base = xcd_tile(blockIdx.x, gridDim.x) * SKG_TILE_T + (threadIdx.x & ~63);
@@ -1072,58 +1112,280 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_cover_lists(const float4 *__rest
 	// entries collect in one VGPR, lane n % 64 holding entry n, and go out as
 	// one coalesced store per 64 (cap is a multiple of 64)
 	int buf = 0;
-	auto emit = [&](int idx) {
-		if (lane == (n & 63)) buf = idx;
-		++n;
-		if ((n & 63) == 0 && n <= cap) out[n - 64 + lane] = buf;
-	};
 	while (node) {
 		node = uniform_int(node);
 		const float4 lo = nlo[node], hi = nhi[node];
 		bool need = false;
-		float c = 0.f;
 		if (valid && lo.w >= 0.f && brange_has(hi.w, pb)) {
 			// hardware square root (about 1 ulp): covered by the factor below
-			c = __builtin_amdgcn_sqrtf(lo.w);
-			const float r = c + margin;
+			const float r = __builtin_amdgcn_sqrtf(lo.w) + margin;
 			need = point_box_d2<false>(lo, hi, p.x, p.y, p.z, 0.f) < r * r * 1.000001f;
 		}
 		if (__any(need)) {
 			if (node < nLeaf2) { node = 2 * node; continue; }
-			if (!ELIST) {
-				emit(node - nLeaf2);
-			} else if (n <= cap) {
-				// An entity of ball r is listed when its reach r + margin holds
-				// the lane's point.  With c the leaf's largest live ball radius,
-				// (r + m)^2 <= r^2 (1 + m/c) + m (c + m) for any c > 0 (since
-				// r^2/c + c >= 2r), so one fma per entity replaces a square
-				// root; the bound is exact for the leaf's largest ball.
-				c = fmaxf(c, 1e-30f);
-				const float k1 = fmaf(margin, 1.f / c, 1.f) * 1.000002f;
-				const float k2 = margin * (c + margin) * 1.000002f;
-				const int2 rg = leaf_range(lstart, node - nLeaf2, B, ne);
-				const int start = uniform_int(rg.x), cnt = uniform_int(rg.y - rg.x);
-				for (int t0 = 0; t0 < cnt; t0 += 4) {
-					// four records per scalar load (the arrays carry SKG_EPAD spare records)
-					float4 A4[4], X4[4];
-#pragma unroll
-					for (int u = 0; u < 4; ++u) { A4[u] = epos[start + t0 + u]; X4[u] = eaux[start + t0 + u]; }
-#pragma unroll
-					for (int u = 0; u < 4; ++u) {
-						if (t0 + u >= cnt) break;
-						if (X4[u].x < 0.f) continue;          // cut (or filler): never hit again
-						const float dx = fsub(A4[u].x, p.x), dy = fsub(A4[u].y, p.y), dz = fsub(A4[u].z, p.z);
-						const bool hit = need && sq3(dx, dy, dz) < fmaf(X4[u].x, k1, k2);
-						if (__any(hit)) emit(start + t0 + u);
-					}
-				}
-			}
+			if (lane == (n & 63)) buf = node - nLeaf2;
+			++n;
+			if ((n & 63) == 0 && n <= cap) out[n - 64 + lane] = buf;
 		}
 		node = (node >> __builtin_ctz(~node)) + 1;
 		if (node == 1) node = 0;
 	}
 	const int rem = n & 63;
 	if (n <= cap && rem && lane < rem) out[n - rem + lane] = buf;
+	if (lane == 0) tcnt[tile] = n <= cap ? n : -1;
+}
+
+// Entity lists: every live entity whose widened reach holds a lane's point, in
+// tree order (so a lane's hits and sums keep the walk's order).  The walk tests
+// 64 nodes at a time (k_cover_wave's frontier) against the tile's bounding box,
+// and the leaves, or any frontier longer than WV_SIFT, against the points,
+// 64 / B leaves are read in a round, a lane per entity, the live ones packed
+// 64 to a window, and each window is tested as the steps do (win_masks; the
+// widened reach in place of the ball), so that the tile's lanes decide on each
+// entity in five operations.  Against the pre-order walk that tested a node at
+// a time and an entity in nine operations and a branch, the bound is the
+// entities under the tile's leaves, about 2.5 for each one listed.
+//
+// A lane within wsteps steps of exactly one face (periodic) may cross it during
+// the block: the list then also holds what reaches the lane's image across that
+// face (with the full margin), and mwrap records the axis (1 + axis), so that a
+// crossing of that face leaves the list valid.  A lane near two or more faces
+// gets code 4, one near none 0: then any crossing sends its wavefront to the
+// tree walk.
+#define WV_F 256              // nodes a wavefront's frontier holds
+#define WV_SIFT 32            // a longer frontier is tested against the points themselves
+__global__ __launch_bounds__(SKG_TILE_T) void k_tile_lists(const float4 *__restrict__ ppos,
+		const int *__restrict__ plist, int np, const float4 *__restrict__ epos, const float4 *__restrict__ eaux, int ne,
+		const float4 *__restrict__ nlo, const float4 *__restrict__ nhi, int nLeaf2, int B,
+		const int *__restrict__ lstart, const int *__restrict__ pbox, const DevBox *__restrict__ bt, int micro,
+		float msteps, float mabs, int per, float wsteps, float cx, float cy, float cz, float Lx, float Ly, float Lz,
+		int cap, int *__restrict__ tlist, int *__restrict__ tcnt, const int *__restrict__ npDev,
+		int *__restrict__ mwrap) {
+	constexpr int NW = SKG_TILE_T / 64;
+	__shared__ int s_fr[NW][2][WV_F];
+	__shared__ float4 s_T[NW][128];
+	__shared__ int s_E[NW][128];
+	__shared__ float4 s_P[NW][64];                // the lanes' points; w: the box's bits
+	if (npDev) np = *npDev;
+	const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+	const int base = xcd_tile(blockIdx.x, gridDim.x) * SKG_TILE_T + (threadIdx.x & ~63);
+	if (base >= np) return;                       // whole wavefront past the end
+	const int tile = base >> 6;
+	const int ii = base + lane;
+	const bool valid = ii < np;
+	const int pi = plist ? plist[valid ? ii : base] : (valid ? ii : base);
+	const float4 p = ppos[pi];
+	const int pb = pbox ? pbox[pi] : 0;
+	const float fStep = micro ? bt[pb].fMicro : bt[pb].fStep;
+	const float mg = wave_max(fmaf(msteps, fStep, mabs));   // the widest margin serves the tile
+	float4 q = p;
+	int code = 0;
+	if (per) {
+		const float cc[3] = {cx, cy, cz}, LL[3] = {Lx, Ly, Lz}, pp[3] = {p.x, p.y, p.z};
+		const float wm = fmaf(wsteps, fStep, mabs);
+		float qq[3] = {p.x, p.y, p.z};
+		int nf = 0;
+#pragma unroll
+		for (int j = 0; j < 3; ++j) {
+			const float h = 0.5f * LL[j];
+			if (pp[j] + wm > cc[j] + h) { qq[j] = pp[j] - LL[j]; code = 1 + j; ++nf; }
+			if (pp[j] - wm <= cc[j] - h) { qq[j] = pp[j] + LL[j]; code = 1 + j; ++nf; }
+		}
+		if (nf > 1) code = 4;
+		if (code >= 1 && code <= 3) q = make_float4(qq[0], qq[1], qq[2], p.w);
+	}
+	const bool img = valid && code >= 1 && code <= 3, wimg = __any(img);
+	if (valid && mwrap) mwrap[pi] = code;
+	const float4 o = make_float4(__shfl(p.x, 32, 64), __shfl(p.y, 32, 64), __shfl(p.z, 32, 64), 0.f);
+	const float4 never = make_float4(0.f, 0.f, 0.f, INFINITY);
+	const float4 w = valid ? win_point(p, o) : never, wq = img ? win_point(q, o) : never;
+	const float3 blo = make_float3(wave_min(p.x), wave_min(p.y), wave_min(p.z));
+	const float3 bhi = make_float3(wave_max(p.x), wave_max(p.y), wave_max(p.z));
+	float3 ilo = blo, ihi = bhi;
+	if (wimg) {
+		ilo = make_float3(wave_min(img ? q.x : INFINITY), wave_min(img ? q.y : INFINITY), wave_min(img ? q.z : INFINITY));
+		ihi = make_float3(wave_max(img ? q.x : -INFINITY), wave_max(img ? q.y : -INFINITY),
+				wave_max(img ? q.z : -INFINITY));
+	}
+	const int wb0 = pbox ? wave_min_i(pb) : 0, wb1 = pbox ? wave_max_i(pb) : 0;
+	const unsigned long long below = (1ull << lane) - 1ull;
+	int n = 0, nw = 0;                            // entries listed; entities in the window
+	int *out = tlist + (size_t)tile * cap, *sE = s_E[wv];
+	float4 *sT = s_T[wv];
+	auto open = [&](int node) {
+		const float4 lo = nlo[node], hi = nhi[node];
+		if (!(lo.w >= 0.f) || !brange_meets(hi.w, wb0, wb1)) return false;
+		// hardware square root (about 1 ulp): covered by the factor below
+		const float r = __builtin_amdgcn_sqrtf(lo.w) + mg, r2 = r * r * 1.000001f;
+		return box_box_d2<false>(lo, hi, blo, bhi, 0.f) < r2 || (wimg && box_box_d2<false>(lo, hi, ilo, ihi, 0.f) < r2);
+	};
+	s_P[wv][lane] = make_float4(p.x, p.y, p.z, __int_as_float(pb));
+	const unsigned long long mimg = __ballot(img);
+	// whether the node (one per lane) reaches any lane's point or image
+	auto reaches = [&](int node) {
+		const float4 lo = nlo[node], hi = nhi[node];
+		const float r = __builtin_amdgcn_sqrtf(fmaxf(lo.w, 0.f)) + mg, r2 = r * r * 1.000001f;
+		auto gap2 = [&](float x, float y, float z) {
+			const float gx = fmaxf(fmaxf(lo.x - x, x - hi.x), 0.f), gy = fmaxf(fmaxf(lo.y - y, y - hi.y), 0.f);
+			const float gz = fmaxf(fmaxf(lo.z - z, z - hi.z), 0.f);
+			return fmaf(gx, gx, fmaf(gy, gy, gz * gz));
+		};
+		bool any = false;
+		if (wb0 == wb1) {
+			for (int t0 = 0; t0 < 64 && !__all(any); t0 += 16)
+#pragma unroll
+				for (int t = t0; t < t0 + 16; ++t) any |= gap2(s_P[wv][t].x, s_P[wv][t].y, s_P[wv][t].z) < r2;
+		} else {
+			for (int t = 0; t < 64; ++t) {
+				const float4 P = s_P[wv][t];
+				any |= gap2(P.x, P.y, P.z) < r2 && brange_has(hi.w, __float_as_int(P.w));
+			}
+		}
+		for (unsigned long long b = mimg; b && !__all(any); b &= b - 1) {
+			const int t = __builtin_ctzll(b);
+			any |= gap2(__shfl(q.x, t, 64), __shfl(q.y, t, 64), __shfl(q.z, t, 64)) < r2 &&
+					brange_has(hi.w, __builtin_amdgcn_readlane(pb, t));
+		}
+		return any;
+	};
+	// the nodes of frontier c that do: into the other buffer; returns their number
+	auto sift = [&](int c, int cnt) {
+		const int *src = s_fr[wv][c];
+		int *dst = s_fr[wv][c ^ 1], nf = 0;
+		wave_lds_sync();
+		for (int t0 = 0; t0 < cnt; t0 += 64) {
+			const int t = t0 + lane, node = src[min(t, cnt - 1)];
+			const bool ok = reaches(node) && t < cnt;
+			const unsigned long long m = __ballot(ok);
+			if (ok) dst[nf + __popcll(m & below)] = node;
+			nf += __popcll(m);
+		}
+		return nf;
+	};
+	// list what the lanes need of the window's first cnt entities (at most 64)
+	auto test = [&](int cnt) {
+		if (lane >= cnt) sT[lane] = make_float4(0.f, 0.f, 0.f, -INFINITY);
+		wave_lds_sync();
+		unsigned m0, m1;
+		win_masks(sT, cnt, w, m0, m1);
+		if (wimg) {
+			unsigned k0, k1;
+			win_masks(sT, cnt, wq, k0, k1);
+			m0 |= k0;
+			m1 |= k1;
+		}
+		m0 = wave_or(m0);
+		m1 = wave_or(m1);
+		const bool on = ((lane < 32 ? m0 : m1) >> (31 - (lane & 31)) & 1u) != 0 && lane < cnt;
+		const unsigned long long b = __ballot(on);
+		if (n + __popcll(b) <= cap) {
+			if (on) out[n + __popcll(b & below)] = sE[lane];
+			n += __popcll(b);
+		} else {
+			n = cap + 1;
+		}
+		wave_lds_sync();
+	};
+	const int bp = B >= 64 ? 64 : (B <= 1 ? 1 : 1 << (32 - __clz(B - 1)));
+	// the entities of a round (in: the lane has one)
+	auto add = [&](int e, bool in) {
+		float4 A, X;
+		if (in) { A = epos[e]; X = eaux[e]; in = X.x >= 0.f; }
+		const unsigned long long b = __ballot(in);
+		if (in) {
+			const int t = nw + __popcll(b & below);
+			const float r = __builtin_amdgcn_sqrtf(X.x) + mg;
+			sT[t] = win_record(A, r * r * 1.000002f, o);
+			sE[t] = e;
+		}
+		nw += __popcll(b);
+		if (nw < 64) return;
+		test(64);
+		nw -= 64;
+		const float4 T = sT[64 + lane];
+		const int E = sE[64 + lane];
+		wave_lds_sync();
+		if (lane < nw) { sT[lane] = T; sE[lane] = E; }
+	};
+	// the entities of the nl leaves whose nodes are in s_fr[wv][c], in order
+	auto scan = [&](int c, int nl) {
+		int *fs = s_fr[wv][c], *fe = s_fr[wv][c ^ 1];
+		wave_lds_sync();
+		for (int t = lane; t < nl; t += 64) {
+			const int2 rg = leaf_range(lstart, fs[t] - nLeaf2, B, ne);
+			fs[t] = rg.x; fe[t] = rg.y;
+		}
+		wave_lds_sync();
+		if (B <= 64) {
+			const int lpr = 64 / bp, g = lane / bp, off = lane & (bp - 1);
+			for (int t0 = 0; t0 < nl && n <= cap; t0 += lpr) {
+				const int t = t0 + g, e = t < nl ? fs[t] + off : 0;
+				add(e, t < nl && e < fe[t]);
+			}
+		} else {
+			for (int t = 0; t < nl; ++t)
+				for (int e0 = fs[t]; e0 < fe[t] && n <= cap; e0 += 64) add(e0 + lane, e0 + lane < fe[t]);
+		}
+		wave_lds_sync();
+	};
+	const int depth = __builtin_ctz(nLeaf2);
+	int lev = min(depth, 6), f, cur = 0;
+	bool over = false;
+	{
+		const bool ok = lane < (1 << lev) && open((1 << lev) + lane);
+		const unsigned long long m = __ballot(ok);
+		if (ok) s_fr[wv][0][__popcll(m & below)] = (1 << lev) + lane;
+		f = __popcll(m);
+	}
+	while (lev < depth && f > 0 && !over) {
+		int d = 1;
+		while (d < depth - lev && (f << (d + 1)) <= 64) ++d;
+		const int tot = f << d;
+		const int *src = s_fr[wv][cur];
+		int *dst = s_fr[wv][cur ^ 1], nf = 0;
+		wave_lds_sync();
+		for (int t0 = 0; t0 < tot; t0 += 64) {
+			const int t = t0 + lane;
+			const int node = t < tot ? (src[t >> d] << d) + (t & ((1 << d) - 1)) : 0;
+			const bool ok = t < tot && open(node);
+			const unsigned long long m = __ballot(ok);
+			const int c = __popcll(m);
+			if (nf + c > WV_F) { over = true; break; }     // even so: the pre-order walk
+			if (ok) dst[nf + __popcll(m & below)] = node;
+			nf += c;
+		}
+		f = nf;
+		lev += d;
+		cur ^= 1;
+		// a tile whose movers lie apart (a jump of the curve, movers that have
+		// crossed a face) has a bounding box that opens far too much
+		if (!over && f > (lev < depth ? WV_SIFT : 0)) { f = sift(cur, f); cur ^= 1; }
+	}
+	if (!over) {
+		if (f > 0) scan(cur, f);
+	} else {
+		int node = 1, nl = 0;
+		wave_lds_sync();
+		while (node && n <= cap) {
+			node = uniform_int(node);
+			bool ok = open(node);
+			if (ok) {                             // exactly, lane by lane
+				const float4 lo = nlo[node], hi = nhi[node];
+				const float r = __builtin_amdgcn_sqrtf(lo.w) + mg, r2 = r * r * 1.000001f;
+				ok = __any(brange_has(hi.w, pb) && (point_box_d2<false>(lo, hi, p.x, p.y, p.z, 0.f) < r2 ||
+						(img && point_box_d2<false>(lo, hi, q.x, q.y, q.z, 0.f) < r2)));
+			}
+			if (ok && node < nLeaf2) { node = 2 * node; continue; }
+			if (ok) {
+				if (lane == 0) s_fr[wv][0][nl] = node;
+				if (++nl == WV_F) { scan(0, nl); nl = 0; }
+			}
+			node = (node >> __builtin_ctz(~node)) + 1;
+			if (node == 1) node = 0;
+		}
+		if (nl) scan(0, nl);
+	}
+	if (nw > 0 && n <= cap) test(nw);
 	if (lane == 0) tcnt[tile] = n <= cap ? n : -1;
 }
 
@@ -1145,8 +1407,8 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 	if (npDev) np = *npDev;                       // device-resident active count and step stamp
 	if (stampDev) stamp = *stampDev;
 	// staging slots for the entity-list scan, 64 per wavefront
-	__shared__ float4 s_eA[SKG_TILE_T], s_eX[SKG_TILE_T];
-	__shared__ int s_eK[SKG_TILE_T], s_eE[SKG_TILE_T];
+	__shared__ float4 s_eA[SKG_TILE_T], s_eX[SKG_TILE_T], s_eT[MODE == 1 ? SKG_TILE_T : 1];
+	__shared__ int s_eK[SKG_TILE_T];
 	const int lane = threadIdx.x & 63;
 	const int base = xcd_tile(blockIdx.x, gridDim.x) * SKG_TILE_T + (threadIdx.x & ~63);
 	if (base >= np) return;                       // whole wavefront past the end
@@ -1161,7 +1423,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 	const bool dl = MODE == 0 && out_dl != nullptr;
 	const float cut = MODE == 1 ? cut_level(cutSlots, nBox, nCut, pb) : 0.f;
 	// With a leaf list for this tile (built at the start of the block, see
-	// k_cover_lists) the wavefront scans those leaves and walks no tree.
+	// k_leaf_lists) the wavefront scans those leaves and walks no tree.
 	// Otherwise a node is opened when its largest live ball reaches at least
 	// one lane's own point (so scattered blocks late in the move loop walk
 	// only the union of their lanes' paths).  The node index is wave-uniform,
@@ -1172,59 +1434,58 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 	// far side, which the list does not cover: the wavefront walks the tree
 	if (nl >= 0 && mwrap && __any(valid && (mwrap[pi] & MWRAP_OUT) != 0)) nl = -1;
 	int node = nl >= 0 ? 0 : 1;
-	if (elist && nl > 0) {
-		// entity list (k_cover_lists<true>): the listed entities in tree
-		// order; a tile that straddles two boxes lists entities of both, and a
-		// lane takes only its own box's range of the entity array (that test
-		// only in such a tile).  The list is staged 64 entries at a time in
-		// this wavefront's slots of LDS: lane j gathers entry j's records
-		// (one coalesced index read, record reads near one another in tree
-		// order), then every lane reads each staged record at one address, a
-		// broadcast.  The wavefront reads back only what it wrote itself, and
-		// LDS operations of one wavefront complete in order.
+	if (MODE == 1 && elist && nl > 0) {
+		// entity list (k_tile_lists): the listed entities in tree order, 64 at a
+		// time in this wavefront's slots of LDS (lane j gathers entry j's
+		// records).  Each lane first marks the entries its point may lie in
+		// (win_masks), then works through its own marks, lane by lane at
+		// different entries: the hit path runs as often as the lane with the
+		// most marks needs it, about 90 times for a list of 400, instead of once
+		// for each of the 320 entries that some lane hits.  The wavefront reads
+		// back only what it wrote itself, and LDS operations of one wavefront
+		// complete in order.
 		const int *L = tlist + (size_t)tile * tcap;
-		int elo = 0, ehi = 0x7FFFFFFF;
-		if (pbox) { elo = eblk[pb] * 256; ehi = eblk[pb + 1] * 256; }
+		int elo = 0, ehi = 0x7FFFFFFF;             // a tile that straddles boxes lists entities of each
+		const bool straddle = pbox && __any(valid && pb != uniform_int(pb));
+		if (straddle) { elo = eblk[pb] * 256; ehi = eblk[pb + 1] * 256; }
 		const int wb = threadIdx.x & ~63;
-		auto scan_list = [&](auto straddle) {
-			for (int c = 0; c < nl; c += 64) {
-				const int m = min(64, nl - c);
-				if (lane < m) {
-					const int e = L[c + lane];
-					s_eA[threadIdx.x] = epos[e];
-					s_eX[threadIdx.x] = eaux[e];
-					s_eK[threadIdx.x] = COMP ? ecode[e] : 13;
-					s_eE[threadIdx.x] = e;
-				}
-				__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-				__builtin_amdgcn_wave_barrier();
-				__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-				for (int j = 0; j < m; j += 2) {
-					float4 A2[2], X2[2];
-					int K2[2], E2[2];
-#pragma unroll
-					for (int u = 0; u < 2; ++u) {
-						A2[u] = s_eA[wb + j + u]; X2[u] = s_eX[wb + j + u];
-						K2[u] = s_eK[wb + j + u]; E2[u] = s_eE[wb + j + u];
-					}
-#pragma unroll
-					for (int u = 0; u < 2; ++u) {
-						if (j + u >= m) break;
-						const int e = E2[u];
-						const bool mine = decltype(straddle)::value ? (valid && e >= elo && e < ehi) : valid;
-						cover_hit<MODE, COMP>(e, A2[u], X2[u], K2[u], mine, p, eorg, ehit, stamp, hmin, Lx, Ly, Lz,
-								s0, s1, s2, false, cut);
-					}
-				}
-				// every lane has read this chunk before the next overwrites it
-				__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-				__builtin_amdgcn_wave_barrier();
-				__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+		const float4 o = make_float4(__shfl(p.x, 32, 64), __shfl(p.y, 32, 64), __shfl(p.z, 32, 64), 0.f);
+		const float4 w = win_point(p, o);
+		int en = lane < nl ? L[lane] : -1;
+		for (int c = 0; c < nl; c += 64) {
+			const int e = en;
+			float4 A = make_float4(0.f, 0.f, 0.f, 0.f), X = make_float4(-1.f, 0.f, 0.f, 0.f);
+			int K = 13;
+			if (e >= 0) {
+				A = epos[e];
+				X = eaux[e];
+				if (COMP) K = ecode[e];
 			}
-		};
-		const int pb0 = uniform_int(pb);
-		if (__any(valid && pb != pb0)) scan_list(std::true_type());
-		else scan_list(std::false_type());
+			en = c + 64 + lane < nl ? L[c + 64 + lane] : -1;
+			s_eT[threadIdx.x] = win_record(A, X.x, o);
+			s_eA[threadIdx.x] = A;
+			s_eX[threadIdx.x] = X;
+			s_eK[threadIdx.x] = K == 13 ? e : ~e;     // a replica's code comes with its source record
+			wave_lds_sync();
+			unsigned m0, m1;
+			win_masks(s_eT + wb, nl - c, w, m0, m1);
+			if (!valid) m0 = m1 = 0;
+			while (__any((m0 | m1) != 0)) {
+				if (m0 | m1) {
+					const bool first = m0 != 0;
+					const int b = __clz(first ? m0 : m1), t = wb + (first ? b : 32 + b);
+					const unsigned keep = ~(0x80000000u >> b);
+					if (first) m0 &= keep;
+					else m1 &= keep;
+					const float4 At = s_eA[t], Xt = s_eX[t];
+					const int Et = s_eK[t], et = Et < 0 ? ~Et : Et;
+					const bool mine = !straddle || (et >= elo && et < ehi);
+					cover_hit<MODE, COMP, true>(et, At, Xt, Et < 0 ? -1 : 13, mine, p, eorg, ehit, stamp, hmin, Lx, Ly, Lz,
+							s0, s1, s2, false, cut);
+				}
+			}
+			wave_lds_sync();                          // every lane has read this chunk
+		}
 	}
 	for (int k = 0; !elist && k < nl; ++k) {
 		const int leaf = uniform_int(tlist[(size_t)tile * tcap + k]);
@@ -1267,142 +1528,6 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 			Ly, Lz, mwrap);
 }
 
-// The first step of a 5-step block with its tile's entity list built on the
-// way: one walk with the block's margin does what k_cover_lists<true> and
-// k_cover<1> would do in two.  A leaf is opened when its largest live ball,
-// widened by the lane's margin, reaches a lane's point; each live entity in it
-// is listed when its own widened reach holds a lane's point (the same fma
-// bound as k_cover_lists<true>), and it adds to a lane's gradient when its
-// ball holds the lane's point.  The widened test opens every node the plain
-// walk opens (and more, whose entities hold no lane's point), and both visit
-// leaves in tree order, so the hits and the order of the sums are k_cover's.
-// Then the lanes' points move.  The list and count go to tlist / tcnt as
-// k_cover_lists<true> writes them.
-template <bool COMP>
-__global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_cover_build(
-		float4 *__restrict__ ppos, const int *__restrict__ plist, int np, const float4 *__restrict__ epos,
-		const float4 *__restrict__ eaux, const float4 *__restrict__ eorg, const int *__restrict__ ecode, int ne,
-		const float4 *__restrict__ nlo, const float4 *__restrict__ nhi, int nLeaf2, int B, int *__restrict__ ehit,
-		int *__restrict__ bthr, const int *__restrict__ pbox, const DevBox *__restrict__ bt, int micro,
-		float msteps, float mabs, int per, float wsteps, float cx, float cy, float cz, float Lx, float Ly,
-		float Lz, const int *__restrict__ lstart, int cap, int *__restrict__ tlist, int *__restrict__ tcnt,
-		const int *__restrict__ npDev, const int *__restrict__ stampDev, int *__restrict__ mwrap) {
-	if (npDev) np = *npDev;
-	const int stamp = stampDev ? *stampDev : 0;
-	// staging slots for an opened leaf's entity records, 64 per wavefront
-	__shared__ float4 s_bA[SKG_TILE_T], s_bX[SKG_TILE_T];
-	__shared__ int s_bK[SKG_TILE_T];
-	const int lane = threadIdx.x & 63;
-	const int base = xcd_tile(blockIdx.x, gridDim.x) * SKG_TILE_T + (threadIdx.x & ~63);
-	if (base >= np) return;                       // whole wavefront past the end
-	const int tile = base >> 6;
-	const int wb = threadIdx.x & ~63;
-	const int ii = base + lane;
-	const bool valid = ii < np;
-	const int pi = plist ? plist[valid ? ii : base] : (valid ? ii : base);
-	const float4 p = ppos[pi];
-	const int pb = pbox ? pbox[pi] : 0;
-	const float fStep = micro ? bt[pb].fMicro : bt[pb].fStep;
-	const float margin = fmaf(msteps, fStep, mabs);
-	// A lane within wsteps steps of exactly one face (periodic) may cross it
-	// during the block: the list then also holds what reaches the lane's image
-	// q across that face (with the full margin), and mwrap records the axis
-	// (1 + axis), so that a crossing of that face leaves the list valid.  A
-	// lane near two or more faces gets code 4, one near none 0: then any
-	// crossing sends its wavefront to the tree walk.
-	float4 q = p;
-	int code = 0;
-	if (per) {
-		const float cc[3] = {cx, cy, cz}, LL[3] = {Lx, Ly, Lz}, pp[3] = {p.x, p.y, p.z};
-		const float wm = fmaf(wsteps, fStep, mabs);
-		float qq[3] = {p.x, p.y, p.z};
-		int nf = 0;
-#pragma unroll
-		for (int j = 0; j < 3; ++j) {
-			const float h = 0.5f * LL[j];
-			if (pp[j] + wm > cc[j] + h) { qq[j] = pp[j] - LL[j]; code = 1 + j; ++nf; }
-			if (pp[j] - wm <= cc[j] - h) { qq[j] = pp[j] + LL[j]; code = 1 + j; ++nf; }
-		}
-		if (nf > 1) code = 4;
-		if (code >= 1 && code <= 3) q = make_float4(qq[0], qq[1], qq[2], p.w);
-	}
-	const bool img = valid && code >= 1 && code <= 3;
-	const bool wimg = __any(img);
-	if (valid && mwrap) mwrap[pi] = code;
-	Sum<COMP> s0, s1, s2;
-	s0.init(); s1.init(); s2.init();
-	float hmin = INFINITY;
-	int n = 0, node = 1;
-	int *out = tlist + (size_t)tile * cap;
-	int buf = 0;                                   // entry n in lane n % 64, stored 64 at a time
-	auto emit = [&](int idx) {
-		if (lane == (n & 63)) buf = idx;
-		++n;
-		if ((n & 63) == 0 && n <= cap) out[n - 64 + lane] = buf;
-	};
-	while (node) {
-		node = uniform_int(node);
-		const float4 lo = nlo[node], hi = nhi[node];
-		bool need = false;
-		float c = 0.f;
-		if (valid && lo.w >= 0.f && brange_has(hi.w, pb)) {
-			// hardware square root (about 1 ulp): covered by the factor below
-			c = __builtin_amdgcn_sqrtf(lo.w);
-			const float r = c + margin, r2 = r * r * 1.000001f;
-			need = point_box_d2<false>(lo, hi, p.x, p.y, p.z, 0.f) < r2;
-			if (wimg && img && !need) need = point_box_d2<false>(lo, hi, q.x, q.y, q.z, 0.f) < r2;
-		}
-		if (__any(need)) {
-			if (node < nLeaf2) { node = 2 * node; continue; }
-			c = fmaxf(c, 1e-30f);
-			const float k1 = fmaf(margin, 1.f / c, 1.f) * 1.000002f;
-			const float k2 = margin * (c + margin) * 1.000002f;
-			const int2 rg = leaf_range(lstart, node - nLeaf2, B, ne);
-			const int start = uniform_int(rg.x), cnt = uniform_int(rg.y - rg.x);
-			// the leaf's records staged in this wavefront's LDS slots, 64 at a
-			// time (lane j reads record j: one round trip), then read by every
-			// lane at one address; the wavefront reads back only what it wrote,
-			// and its LDS operations complete in order
-			for (int c0 = 0; c0 < cnt; c0 += 64) {
-				const int m = min(64, cnt - c0);
-				if (lane < m) {
-					s_bA[threadIdx.x] = epos[start + c0 + lane];
-					s_bX[threadIdx.x] = eaux[start + c0 + lane];
-					s_bK[threadIdx.x] = COMP ? ecode[start + c0 + lane] : 13;
-				}
-				__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-				__builtin_amdgcn_wave_barrier();
-				__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-				for (int t = 0; t < m; ++t) {
-					const float4 A = s_bA[wb + t], X = s_bX[wb + t];
-					if (X.x < 0.f) continue;              // cut (or filler): neither listed nor hit
-					const int e = start + c0 + t;
-					const float dx = fsub(A.x, p.x), dy = fsub(A.y, p.y), dz = fsub(A.z, p.z);
-					const float reach = fmaf(X.x, k1, k2);
-					bool listed = need && sq3(dx, dy, dz) < reach;
-					if (wimg && img && need && !listed)
-						listed = sq3(fsub(A.x, q.x), fsub(A.y, q.y), fsub(A.z, q.z)) < reach;
-					if (__any(listed)) emit(e);
-					cover_hit<1, COMP>(e, A, X, s_bK[wb + t], need, p, eorg, ehit, stamp, hmin, Lx, Ly, Lz, s0, s1,
-							s2);
-				}
-				// every lane has read these records before the next chunk overwrites them
-				__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-				__builtin_amdgcn_wave_barrier();
-				__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-			}
-		}
-		node = (node >> __builtin_ctz(~node)) + 1;
-		if (node == 1) node = 0;
-	}
-	const int rem = n & 63;
-	if (n <= cap && rem && lane < rem) out[n - rem + lane] = buf;
-	if (lane == 0) tcnt[tile] = n <= cap ? n : -1;
-	if (bthr) box_min_atomic(hmin, valid, pb, bthr);
-	if (!valid) return;
-	move_point(ppos, pi, p, s0.val(), s1.val(), s2.val(), fStep, cx, cy, cz, Lx, Ly, Lz, mwrap);
-}
-
 // One wavefront per point, for point sets too small (or too scattered) to fill
 // the card with a lane per point.  The walk tests 64 nodes at a time: the
 // frontier of opened nodes sits in LDS in tree order, and each round tests the
@@ -1425,14 +1550,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 //
 // A frontier of more than WV_F nodes (very large balls) falls back to the
 // pre-order walk, its leaves taken WV_F at a time.
-#define WV_F 256
 #define WV_Q 256              // queued terms per wavefront: WV_Q / S' per lane j
-__device__ __forceinline__ void wave_lds_sync() {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <int MODE, bool COMP, int S>
 __global__ __launch_bounds__(SKG_TILE_T) void k_cover_wave(
 		float4 *__restrict__ ppos, const int *__restrict__ plist, int np,
@@ -2280,7 +2398,6 @@ extern "C" int skg_create(const skg_params *P, skg_ctx **out) {
 	if (const char *e = getenv("SKG_COVER_S64_MAX")) c->s64Max = atol(e);
 	if (const char *e = getenv("SKG_KNN_BUCKET")) c->knnBucket = std::max(0, std::min(1024, atoi(e)));
 	if (const char *e = getenv("SKG_KNN_WAVES")) c->knnWaves = atoi(e) == 2 ? 2 : 1;
-	if (const char *e = getenv("SKG_FUSED_BUILD")) c->fusedBuild = atoi(e) != 0;
 	if (const char *e = getenv("SKG_TILE_LISTS")) c->useLists = atoi(e);
 	c->tlCap = c->useLists == 2 ? 512 : 1024;
 	if (const char *e = getenv("SKG_TILE_CAP")) { c->tlCap = std::max(4, atoi(e) & ~3); c->tlCapFixed = 1; }
@@ -2705,20 +2822,25 @@ static int count_active(skg_ctx *c, long cap) {
 	return 0;
 }
 
-// Leaf lists for the next nsteps steps (margin: the distance a mover can
-// travel before the last of them, nsteps - 1 steps of its own box's step, a
-// lane at a time: step i takes its gradient at the point i moves away).
+// Lists for the next nsteps steps (margin: the distance a mover can travel
+// before the last of them, nsteps - 1 steps of its own box's step: step i takes
+// its gradient at the point i moves away).  Lanes within nsteps - 2 steps of a
+// face get their image listed too: they can cross it in time for two or more
+// of the block's steps (closer to the margin the build walks more than the
+// steps save).
 static void enqueue_lists(skg_ctx *c, long cap, int nsteps, int micro) {
 	const float mabs = 1e-6f * c->P.fPeriod[0] * (c->P.bPeriodic ? 1.f : 0.f);
 	const float *C = c->P.fCenter, *L = c->P.fPeriod;
-#define LL(E_) k_cover_lists<E_><<<nblk(cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_list, (int)cap,    \
-			c->te.lo, c->te.hi, c->te.nLeaf2, c->nBox > 1 ? c->m_box : nullptr, c->d_bt, micro,                    \
-			1.02f * (nsteps - 1),                                                                                \
-			mabs, c->P.bPeriodic, C[0], C[1], C[2], L[0], L[1], L[2], c->tlCap, c->tl_list, c->tl_cnt,          \
-			c->d_ml + 1, c->e_pos, c->e_aux, c->te.lstart, c->te.B, c->nE, c->m_wrap)
-	if (c->useLists == 2) LL(false);
-	else LL(true);
-#undef LL
+	const int *pbox = c->nBox > 1 ? c->m_box : nullptr;
+	if (c->useLists == 2)
+		k_leaf_lists<<<nblk(cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_list, (int)cap, c->te.lo, c->te.hi,
+				c->te.nLeaf2, pbox, c->d_bt, micro, 1.02f * (nsteps - 1), mabs, c->tlCap, c->tl_list, c->tl_cnt,
+				c->d_ml + 1, c->m_wrap);
+	else
+		k_tile_lists<<<nblk(cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_list, (int)cap, c->e_pos, c->e_aux,
+				c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, c->te.lstart, pbox, c->d_bt, micro,
+				1.02f * (nsteps - 1), mabs, c->P.bPeriodic, 1.02f * (nsteps - 2), C[0], C[1], C[2], L[0], L[1], L[2],
+				c->tlCap, c->tl_list, c->tl_cnt, c->d_ml + 1, c->m_wrap);
 }
 
 // nsteps Denmax steps over the active list (at most cap movers).
@@ -2732,23 +2854,19 @@ static int enqueue_steps(skg_ctx *c, long cap, bool sub, bool lists, int nsteps,
 	const float *C = c->P.fCenter, *L = c->P.fPeriod;
 	const int *pbox = c->nBox > 1 ? c->m_box : nullptr;
 	const int nb = nblk(c->nE, 256);
-	const float mabs = 1e-6f * c->P.fPeriod[0] * (c->P.bPeriodic ? 1.f : 0.f);
 	const char *ft = getenv("SKG_FUSED_THR");
 	const bool fusedThr = !(ft && atoi(ft) == 0);
-	// entity lists: built by the block's first step itself (k_cover_build), or
-	// by a pass of their own before it (SKG_FUSED_BUILD=0, and leaf lists)
-	const bool fusedBuild = lists && c->useLists != 2 && c->fusedBuild;
-	// lanes within this many steps of a face get their image listed too: they
-	// can cross it in time for two or more of the block's list steps (closer
-	// to the margin the build walks more than the list steps save)
-	const float wsteps = 1.02f * (nsteps - 2);
 	// With the entities sorted by density, a step's cut is not applied before
 	// the next step: the move kernels skip what lies below the thresholds so
 	// far, and one k_cut_sorted ends the run.  With the one-launch prune and
 	// refit a block of five steps over a small list is 8 launches (31 before),
 	// a whole pass 10.7 -> 8.7 ms for 2,048 points and 19.4 -> 16.5 for 32,768.
 	const bool lazy = fusedThr && c->cutReady && !bInitial && nsteps <= SKG_BLOCK_STEPS;
-	if (lists && !fusedBuild) enqueue_lists(c, cap, nsteps, micro);
+	if (lists) {
+		const int bslot = capturing ? -1 : skg_prof_begin(c);
+		enqueue_lists(c, cap, nsteps, micro);
+		if (bslot >= 0) skg_prof_end(c, bslot, SKG_K_COVER_BUILD, 24.0 * c->nActive + 24.0 * c->nLive);
+	}
 	for (int i = 0; i < nsteps; ++i) {
 		// the initial step stamps its hits (unhit entities get density 0);
 		// later steps take the threshold from the move kernel itself
@@ -2777,19 +2895,10 @@ static int enqueue_steps(skg_ctx *c, long cap, bool sub, bool lists, int nsteps,
 				ehit, 0, bthr, pbox, c->d_bt, micro, C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart,           \
 				lists ? c->tl_list : nullptr, lists ? c->tl_cnt : nullptr, c->tlCap, c->d_ml + 1, c->d_ml,  \
 				c->useLists != 2, c->d_eblk, nullptr, lists ? c->m_wrap : nullptr, c->d_bslot, c->nBox, nCut)
-#define MB(C_)                                                                                                \
-		k_cover_build<C_><<<nblk(cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_list, (int)cap, c->e_pos, \
-				c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, ehit, bthr, pbox,   \
-				c->d_bt, micro, 1.02f * (nsteps - 1), mabs, c->P.bPeriodic, wsteps, C[0], C[1], C[2], L[0], L[1], L[2], \
-				c->te.lstart,                                                                                        \
-				c->tlCap, c->tl_list, c->tl_cnt, c->d_ml + 1, c->d_ml, c->m_wrap)
-		if (fusedBuild && i == 0) { if (comp) { MB(true); } else { MB(false); } }
-		else if (comp) { MV(true); } else { MV(false); }
-#undef MB
+		if (comp) { MV(true); } else { MV(false); }
 #undef MV
 		if (pslot >= 0)
-			skg_prof_end(c, pslot, fusedBuild && i == 0 ? SKG_K_COVER_BUILD : SKG_K_COVER_MOVE,
-					24.0 * c->nActive + 24.0 * c->nLive);
+			skg_prof_end(c, pslot, SKG_K_COVER_MOVE, 24.0 * c->nActive + 24.0 * c->nLive);
 		if (lazy) continue;
 		if (stamps) {
 			k_scat_thr<<<nb, 256, 0, c->st>>>(c->e_live, c->e_hit, c->e_rho, c->e_aux, c->nE, c->d_ml, bInitial,
