@@ -155,6 +155,7 @@ struct skg_ctx {
 	int *d_ml = nullptr;
 	int *m_flag = nullptr, *m_bcnt = nullptr;   // prune flags; block counts then offsets
 	int *m_wrap = nullptr;                       // per mover: wrapped across a periodic face since its tile's list was built
+	int *m_odd = nullptr;                        // movers without a valid list in this block (their number: ml[3])
 	long lastSort = 0;                          // active count at the last mover sort
 	// ScatterCut over density-sorted entities (after the initial step): each
 	// box's live entities in ascending density, its first still-live position

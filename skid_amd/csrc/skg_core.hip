@@ -1052,11 +1052,13 @@ __device__ __forceinline__ float cut_level(const float *__restrict__ slots, int 
 }
 // kdMoveParticles (kd.c:702-732) for one lane: a step of fStep against the
 // gradient (ax, ay, az), then the periodic wrap into the box; a wrap sets the
-// mover's flag (mwrap) that sends its wavefront back to the tree walk for the
+// mover's flag (mwrap): its tile's list does not hold for it any more, and it
+// joins the odd movers (or sends its wavefront back to the tree walk) for the
 // rest of the block.
 #define MWRAP_OUT 8
 __device__ __forceinline__ void move_point(float4 *__restrict__ ppos, int pi, const float4 &p, float ax, float ay,
-		float az, float fStep, float cx, float cy, float cz, float Lx, float Ly, float Lz, int *__restrict__ mwrap) {
+		float az, float fStep, float cx, float cy, float cz, float Lx, float Ly, float Lz, int *__restrict__ mwrap,
+		int *__restrict__ odd = nullptr, int *__restrict__ nOdd = nullptr) {
 	const float ss = sq3(ax, ay, az);
 	float ai = (float)sqrt((double)ss);
 	if (ai > 0.0f) ai = (float)((double)fStep / sqrt((double)ss));
@@ -1073,7 +1075,10 @@ __device__ __forceinline__ void move_point(float4 *__restrict__ ppos, int pi, co
 	// 0 for none) and gains MWRAP_OUT when the mover crosses another face
 	if (wrapped && mwrap) {
 		const int code = mwrap[pi] & 7;
-		if (code == 0 || code > 3 || (wrapped & ~(1 << (code - 1)))) mwrap[pi] = code | MWRAP_OUT;
+		if (code == 0 || code > 3 || (wrapped & ~(1 << (code - 1)))) {
+			mwrap[pi] = code | MWRAP_OUT;
+			if (odd) odd[atomicAdd(nOdd, 1)] = pi;
+		}
 	}
 }
 
@@ -1081,12 +1086,16 @@ __device__ __forceinline__ void move_point(float4 *__restrict__ ppos, int pi, co
 // removes balls, so while the active list (and with it every tile of 64 movers)
 // is unchanged, what any step can need lies within a ball's reach of a lane's
 // point now, the reach widened by the distance a mover can still travel
-// (margin).  One walk per block then replaces one walk per step.  A tile with
-// more than cap entries gets count -1 and walks the tree.  Near a periodic face
-// the lists include the replicas there; a mover that crosses the face during
-// the block jumps to the far side, which its list may not cover: the move step
-// then flags it (mwrap) and its wavefront walks the tree for the rest of the
-// block.
+// (margin).  One walk per block then replaces one walk per step.  Near a
+// periodic face the lists include the replicas there; a mover that crosses the
+// face during the block jumps to the far side, which its list may not cover:
+// the move step then flags it (mwrap).  What has no valid list -- flagged
+// movers, and tiles with more than cap entries (count -1) -- walks the tree with
+// its wavefront (leaf lists) or, with entity lists, is an odd mover: it leaves
+// its tile and takes the block's steps with a wavefront to itself
+// (k_cover_wave over the odd list, in the order of one lane's sums).  A few such
+// tiles or movers used to hold a whole launch: its length was that of its
+// slowest wavefront, 0.4 to 0.7 ms however few movers were left.
 
 // Leaf lists (SKG_TILE_LISTS=2): the leaves a lane's point can reach.
 __global__ __launch_bounds__(SKG_TILE_T) void k_leaf_lists(const float4 *__restrict__ ppos,
@@ -1153,6 +1162,7 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_leaf_lists(const float4 *__restr
 // gets code 4, one near none 0: then any crossing sends its wavefront to the
 // tree walk.
 #define WV_F 256              // nodes a wavefront's frontier holds
+#define TL_F 512              // the same of a tile: past it the tile is given up (2M gas+dark: 216 ms at 256, 179 at 512, 184 at 1024)
 #define WV_SIFT 32            // a longer frontier is tested against the points themselves
 __global__ __launch_bounds__(SKG_TILE_T) void k_tile_lists(const float4 *__restrict__ ppos,
 		const int *__restrict__ plist, int np, const float4 *__restrict__ epos, const float4 *__restrict__ eaux, int ne,
@@ -1160,9 +1170,9 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_tile_lists(const float4 *__restr
 		const int *__restrict__ lstart, const int *__restrict__ pbox, const DevBox *__restrict__ bt, int micro,
 		float msteps, float mabs, int per, float wsteps, float cx, float cy, float cz, float Lx, float Ly, float Lz,
 		int cap, int *__restrict__ tlist, int *__restrict__ tcnt, const int *__restrict__ npDev,
-		int *__restrict__ mwrap) {
+		int *__restrict__ mwrap, int *__restrict__ odd, int *__restrict__ nOdd) {
 	constexpr int NW = SKG_TILE_T / 64;
-	__shared__ int s_fr[NW][2][WV_F];
+	__shared__ int s_fr[NW][2][TL_F];
 	__shared__ float4 s_T[NW][128];
 	__shared__ int s_E[NW][128];
 	__shared__ float4 s_P[NW][64];                // the lanes' points; w: the box's bits
@@ -1350,7 +1360,7 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_tile_lists(const float4 *__restr
 			const bool ok = t < tot && open(node);
 			const unsigned long long m = __ballot(ok);
 			const int c = __popcll(m);
-			if (nf + c > WV_F) { over = true; break; }     // even so: the pre-order walk
+			if (nf + c > TL_F) { over = true; break; }     // even so: odd movers
 			if (ok) dst[nf + __popcll(m & below)] = node;
 			nf += c;
 		}
@@ -1361,38 +1371,28 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_tile_lists(const float4 *__restr
 		// crossed a face) has a bounding box that opens far too much
 		if (!over && f > (lev < depth ? WV_SIFT : 0)) { f = sift(cur, f); cur ^= 1; }
 	}
-	if (!over) {
-		if (f > 0) scan(cur, f);
-	} else {
-		int node = 1, nl = 0;
-		wave_lds_sync();
-		while (node && n <= cap) {
-			node = uniform_int(node);
-			bool ok = open(node);
-			if (ok) {                             // exactly, lane by lane
-				const float4 lo = nlo[node], hi = nhi[node];
-				const float r = __builtin_amdgcn_sqrtf(lo.w) + mg, r2 = r * r * 1.000001f;
-				ok = __any(brange_has(hi.w, pb) && (point_box_d2<false>(lo, hi, p.x, p.y, p.z, 0.f) < r2 ||
-						(img && point_box_d2<false>(lo, hi, q.x, q.y, q.z, 0.f) < r2)));
-			}
-			if (ok && node < nLeaf2) { node = 2 * node; continue; }
-			if (ok) {
-				if (lane == 0) s_fr[wv][0][nl] = node;
-				if (++nl == WV_F) { scan(0, nl); nl = 0; }
-			}
-			node = (node >> __builtin_ctz(~node)) + 1;
-			if (node == 1) node = 0;
-		}
-		if (nl) scan(0, nl);
-	}
-	if (nw > 0 && n <= cap) test(nw);
-	if (lane == 0) tcnt[tile] = n <= cap ? n : -1;
+	if (!over && f > 0) scan(cur, f);
+	if (!over && nw > 0 && n <= cap) test(nw);
+	over |= n > cap;
+	if (lane == 0) tcnt[tile] = over ? -1 : n;
+	if (!over) return;
+	int at = 0;
+	if (lane == 0) at = atomicAdd(nOdd, min(64, np - base));
+	if (valid) odd[uniform_int(at) + lane] = pi;
 }
 
 // pbox (indexed like ppos; none: box 0) gives each point's box: a lane opens
 // only nodes holding its box, and the entity array starts every box on a new
 // leaf, so every entity a lane tests is of its own box.  MODE 1 takes the
 // box's step (micro: its micro-step).
+// List entries a wavefront holds in LDS at a time.  A longer window evens out
+// what the lanes have to do (13 hit rounds of 64 entries, 22 of 128), but its
+// LDS costs wavefronts: 128 measured 2% slower, 256 20%.
+#define LIST_W 64
+// Entries of a tile's list.  A longer one holds its launch: past it the tile's
+// movers get a wavefront each (48 boxes of 2,048 to 524,288 points, a pass:
+// 184 ms at 2048, 176 at 4096, 177 at 8192).
+#define LIST_CAP 4096
 template <int MODE, bool COMP>
 __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_cover(
 		float4 *__restrict__ ppos, const int *__restrict__ plist, int np,
@@ -1403,20 +1403,27 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		float cx, float cy, float cz, float Lx, float Ly, float Lz, const int *__restrict__ lstart,
 		const int *__restrict__ tlist, const int *__restrict__ tcnt, int tcap, const int *__restrict__ npDev,
 		const int *__restrict__ stampDev, int elist, const int *__restrict__ eblk, float *__restrict__ out_dl,
-		int *__restrict__ mwrap, const float *__restrict__ cutSlots, int nBox, int nCut) {
+		int *__restrict__ mwrap, const float *__restrict__ cutSlots, int nBox, int nCut, int *__restrict__ odd,
+		int *__restrict__ nOdd) {
 	if (npDev) np = *npDev;                       // device-resident active count and step stamp
 	if (stampDev) stamp = *stampDev;
 	// staging slots for the entity-list scan, 64 per wavefront
-	__shared__ float4 s_eA[SKG_TILE_T], s_eX[SKG_TILE_T], s_eT[MODE == 1 ? SKG_TILE_T : 1];
+	constexpr int LW = MODE == 1 ? LIST_W : 64;
+	__shared__ float4 s_eA[SKG_TILE_T / 64 * LW], s_eX[SKG_TILE_T / 64 * LW];
+	__shared__ float4 s_eT[MODE == 1 ? SKG_TILE_T : 1], s_eO[MODE == 1 && COMP ? SKG_TILE_T / 64 * LW : 1];
 	__shared__ int s_eK[SKG_TILE_T];
 	const int lane = threadIdx.x & 63;
 	const int base = xcd_tile(blockIdx.x, gridDim.x) * SKG_TILE_T + (threadIdx.x & ~63);
 	if (base >= np) return;                       // whole wavefront past the end
 	const int ii = base + lane;
-	const bool valid = ii < np;
+	bool valid = ii < np;
 	const int pi = plist ? plist[valid ? ii : base] : (valid ? ii : base);
 	const float4 p = ppos[pi];
 	const int pb = pbox ? pbox[pi] : 0;
+	if (MODE == 1 && odd) {                       // odd movers are not this kernel's
+		if (tcnt[base >> 6] < 0) return;
+		valid = valid && (mwrap[pi] & MWRAP_OUT) == 0;
+	}
 	Sum<COMP> s0, s1, s2;
 	s0.init(); s1.init(); s2.init();
 	float hmin = INFINITY;
@@ -1432,60 +1439,125 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 	int nl = tcnt ? uniform_int(tcnt[tile]) : -1;
 	// a lane that crossed a periodic face since the list was built is on the
 	// far side, which the list does not cover: the wavefront walks the tree
-	if (nl >= 0 && mwrap && __any(valid && (mwrap[pi] & MWRAP_OUT) != 0)) nl = -1;
+	if (nl >= 0 && !odd && mwrap && __any(valid && (mwrap[pi] & MWRAP_OUT) != 0)) nl = -1;
 	int node = nl >= 0 ? 0 : 1;
 	if (MODE == 1 && elist && nl > 0) {
-		// entity list (k_tile_lists): the listed entities in tree order, 64 at a
-		// time in this wavefront's slots of LDS (lane j gathers entry j's
+		// entity list (k_tile_lists): the listed entities in tree order, LIST_W
+		// at a time in this wavefront's slots of LDS (lane j gathers entry j's
 		// records).  Each lane first marks the entries its point may lie in
 		// (win_masks), then works through its own marks, lane by lane at
 		// different entries: the hit path runs as often as the lane with the
-		// most marks needs it, about 90 times for a list of 400, instead of once
-		// for each of the 320 entries that some lane hits.  The wavefront reads
-		// back only what it wrote itself, and LDS operations of one wavefront
-		// complete in order.
+		// most marks needs it, about 13 times for 64 entries, instead of once for
+		// each entry that some lane hits.  It has no branch: a lane without a
+		// mark left, or whose entry the exact test drops, adds zeros (the sums
+		// start at +0, so that changes no bit).  The wavefront reads back only
+		// what it wrote itself, and LDS operations of one wavefront complete in
+		// order.
 		const int *L = tlist + (size_t)tile * tcap;
-		int elo = 0, ehi = 0x7FFFFFFF;             // a tile that straddles boxes lists entities of each
+		const int wv = threadIdx.x >> 6;
+		float4 *sT = s_eT + wv * 64, *sA = s_eA + wv * LW, *sX = s_eX + wv * LW, *sO = s_eO + wv * LW;
+		// a tile that straddles boxes lists entities of each: a lane takes its own box's range
 		const bool straddle = pbox && __any(valid && pb != uniform_int(pb));
-		if (straddle) { elo = eblk[pb] * 256; ehi = eblk[pb + 1] * 256; }
-		const int wb = threadIdx.x & ~63;
+		const int elo = straddle ? eblk[pb] * 256 : 0, ehi = straddle ? eblk[pb + 1] * 256 : 0x7FFFFFFF;
 		const float4 o = make_float4(__shfl(p.x, 32, 64), __shfl(p.y, 32, 64), __shfl(p.z, 32, 64), 0.f);
 		const float4 w = win_point(p, o);
+		unsigned hm = __float_as_uint(INFINITY);      // hmin's bits (densities are >= 0)
 		int en = lane < nl ? L[lane] : -1;
-		for (int c = 0; c < nl; c += 64) {
-			const int e = en;
-			float4 A = make_float4(0.f, 0.f, 0.f, 0.f), X = make_float4(-1.f, 0.f, 0.f, 0.f);
-			int K = 13;
-			if (e >= 0) {
-				A = epos[e];
-				X = eaux[e];
-				if (COMP) K = ecode[e];
-			}
-			en = c + 64 + lane < nl ? L[c + 64 + lane] : -1;
-			s_eT[threadIdx.x] = win_record(A, X.x, o);
-			s_eA[threadIdx.x] = A;
-			s_eX[threadIdx.x] = X;
-			s_eK[threadIdx.x] = K == 13 ? e : ~e;     // a replica's code comes with its source record
-			wave_lds_sync();
-			unsigned m0, m1;
-			win_masks(s_eT + wb, nl - c, w, m0, m1);
-			if (!valid) m0 = m1 = 0;
-			while (__any((m0 | m1) != 0)) {
-				if (m0 | m1) {
-					const bool first = m0 != 0;
-					const int b = __clz(first ? m0 : m1), t = wb + (first ? b : 32 + b);
-					const unsigned keep = ~(0x80000000u >> b);
-					if (first) m0 &= keep;
-					else m1 &= keep;
-					const float4 At = s_eA[t], Xt = s_eX[t];
-					const int Et = s_eK[t], et = Et < 0 ? ~Et : Et;
-					const bool mine = !straddle || (et >= elo && et < ehi);
-					cover_hit<MODE, COMP, true>(et, At, Xt, Et < 0 ? -1 : 13, mine, p, eorg, ehit, stamp, hmin, Lx, Ly, Lz,
-							s0, s1, s2, false, cut);
+		for (int c = 0; c < nl; c += LW) {
+			unsigned m[LW / 32];
+			bool reps = false;                        // a replica among the window's entries
+#pragma unroll
+			for (int u = 0; u < LW / 64; ++u) {
+				m[2 * u] = m[2 * u + 1] = 0;
+				if (c + 64 * u >= nl) continue;
+				const int e = en, nx = c + 64 * (u + 1) + lane;
+				float4 A = make_float4(0.f, 0.f, 0.f, 0.f), X = make_float4(-1.f, 0.f, 0.f, 0.f);
+				int K = 13;
+				if (e >= 0) {
+					A = epos[e];
+					X = eaux[e];
+					if (COMP) K = ecode[e];
 				}
+				en = nx < nl ? L[nx] : -1;
+				if (!straddle && cut_by(X.w, cut)) X.x = -1.f;
+				sT[lane] = win_record(A, X.x, o);
+				A.w = __int_as_float(e);
+				sA[64 * u + lane] = A;
+				sX[64 * u + lane] = X;
+				if (COMP) {
+					const unsigned long long b = __ballot(K != 13);
+					if (b) {                          // source positions and image codes
+						if (!reps && u > 0)
+							for (int v = 0; v < u; ++v) { float4 S = sA[64 * v + lane]; S.w = 13.f; sO[64 * v + lane] = S; }
+						reps = true;
+					}
+					if (reps) {
+						float4 S = A;
+						S.w = 13.f;
+						if (K != 13) S = eorg[e];
+						sO[64 * u + lane] = S;
+					}
+				}
+				wave_lds_sync();
+				win_masks(sT, nl - c - 64 * u, w, m[2 * u], m[2 * u + 1]);
+				wave_lds_sync();
 			}
-			wave_lds_sync();                          // every lane has read this chunk
+			if (!valid)
+#pragma unroll
+				for (int u = 0; u < LW / 32; ++u) m[u] = 0;
+			auto work = [&](auto general) {
+				constexpr bool GEN = decltype(general)::value;
+				for (;;) {
+					unsigned any = 0;
+#pragma unroll
+					for (int u = 0; u < LW / 32; ++u) any |= m[u];
+					if (!__any(any != 0)) break;
+					// the lane's first mark, and the mark taken off
+					unsigned cur = m[LW / 32 - 1];
+					int b0 = LW - 32;
+#pragma unroll
+					for (int u = LW / 32 - 2; u >= 0; --u)
+						if (m[u]) { cur = m[u]; b0 = 32 * u; }
+					const int b = __builtin_clz(cur | 1u);
+					const unsigned keep = ~(0x80000000u >> b);
+					bool before = true;
+#pragma unroll
+					for (int u = 0; u < LW / 32; ++u) {
+						const bool here = before && (m[u] != 0 || u == LW / 32 - 1);
+						m[u] = here ? m[u] & keep : m[u];
+						before = before && !here;
+					}
+					const int t = b0 + b;
+					const float4 A = sA[t], X = sX[t];
+					float dx = fsub(A.x, p.x), dy = fsub(A.y, p.y), dz = fsub(A.z, p.z);
+					float d2 = sq3(dx, dy, dz);
+					bool hit = any != 0 && d2 < X.x;
+					if (GEN) {
+						const int e = __float_as_int(A.w);
+						hit = hit && e >= elo && e < ehi && !cut_by(X.w, cut);
+						if (COMP && reps) {
+							// separation from the source position plus the exact shift (no
+							// shift: the rounded difference itself, bit for bit)
+							const float4 S = sO[t];
+							const int K = (int)S.w;
+							dx = exact_delta(S.x, p.x, (float)(K / 9 - 1) * Lx);
+							dy = exact_delta(S.y, p.y, (float)((K / 3) % 3 - 1) * Ly);
+							dz = exact_delta(S.z, p.z, (float)(K % 3 - 1) * Lz);
+							d2 = sq3(dx, dy, dz);
+						}
+					}
+					float f = COMP ? grad_factor_f32(d2, X.y, X.z) : grad_factor(d2, X.y, X.z);
+					f = hit ? f : 0.f;
+					s0.add(fmul(dx, f)); s1.add(fmul(dy, f)); s2.add(fmul(dz, f));
+					if (ehit && hit) ehit[__float_as_int(A.w)] = stamp;
+					hm = min(hm, hit ? __float_as_uint(X.w) : hm);
+				}
+			};
+			if (reps || straddle) work(std::true_type());
+			else work(std::false_type());
+			wave_lds_sync();                          // every lane has read this window
 		}
+		hmin = __uint_as_float(hm);
 	}
 	for (int k = 0; !elist && k < nl; ++k) {
 		const int leaf = uniform_int(tlist[(size_t)tile * tcap + k]);
@@ -1498,7 +1570,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		if (!__any(want)) continue;
 		const int2 rg = leaf_range(lstart, leaf, B, ne);
 		cover_scan_staged<MODE, COMP>(uniform_int(rg.x), uniform_int(rg.y - rg.x), want, p, epos, eaux, eorg, ecode,
-				ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x & ~63), s_eX + (threadIdx.x & ~63),
+				ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x >> 6) * LW, s_eX + (threadIdx.x >> 6) * LW,
 				s_eK + (threadIdx.x & ~63), lane, cut);
 	}
 	while (node) {
@@ -1510,8 +1582,8 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		if (visit) {
 			const int2 rg = leaf_range(lstart, node - nLeaf2, B, ne);
 			cover_scan_staged<MODE, COMP>(uniform_int(rg.x), uniform_int(rg.y - rg.x), need, p, epos, eaux, eorg,
-					ecode, ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x & ~63),
-					s_eX + (threadIdx.x & ~63), s_eK + (threadIdx.x & ~63), lane, cut);
+					ecode, ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x >> 6) * LW,
+					s_eX + (threadIdx.x >> 6) * LW, s_eK + (threadIdx.x & ~63), lane, cut);
 		}
 		// next node in pre-order after node's subtree (strip trailing ones, step)
 		node = (node >> __builtin_ctz(~node)) + 1;
@@ -1525,7 +1597,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		return;
 	}
 	move_point(ppos, pi, p, s0.val(), s1.val(), s2.val(), micro ? bt[pb].fMicro : bt[pb].fStep, cx, cy, cz, Lx,
-			Ly, Lz, mwrap);
+			Ly, Lz, mwrap, odd, nOdd);
 }
 
 // One wavefront per point, for point sets too small (or too scattered) to fill
@@ -1550,6 +1622,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 //
 // A frontier of more than WV_F nodes (very large balls) falls back to the
 // pre-order walk, its leaves taken WV_F at a time.
+#define ODD_WG 1024           // workgroups of the odd movers' launch
 #define WV_Q 256              // queued terms per wavefront: WV_Q / S' per lane j
 template <int MODE, bool COMP, int S>
 __global__ __launch_bounds__(SKG_TILE_T) void k_cover_wave(
@@ -1567,8 +1640,9 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_cover_wave(
 	if (npDev) np = *npDev;
 	if (stampDev) stamp = *stampDev;
 	const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-	const int ii = uniform_int(xcd_tile(blockIdx.x, gridDim.x) * NW + wv);
-	if (ii >= np) return;                         // no workgroup barrier in this kernel
+	// a launch covers the points once, or (the odd movers' fixed grid) in strides;
+	// no workgroup barrier in this kernel
+	for (int ii = uniform_int(xcd_tile(blockIdx.x, gridDim.x) * NW + wv); ii < np; ii += gridDim.x * NW) {
 	const int pi = plist ? plist[ii] : ii;
 	const float4 p = ppos[pi];
 	const int pb = pbox ? pbox[pi] : 0;
@@ -1735,14 +1809,18 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_cover_wave(
 		if (MODE == 1) s2.xor_merge(o);
 	}
 	if (MODE == 1 && bthr) box_min_atomic(hmin, true, pb, bthr);
-	if (lane != 0) return;
-	if (MODE == 0) {
-		out_sum[ii] = s0.val();
-		if (dl) out_dl[ii] = s1.val() * (float)(-M_1_PI / 6.0);
-		return;
+	if (lane == 0) {
+		if (MODE == 0) {
+			out_sum[ii] = s0.val();
+			if (dl) out_dl[ii] = s1.val() * (float)(-M_1_PI / 6.0);
+		} else {
+			move_point(ppos, pi, p, s0.val(), s1.val(), s2.val(), micro ? bt[pb].fMicro : bt[pb].fStep, cx, cy, cz, Lx,
+					Ly, Lz, nullptr);
+		}
 	}
-	move_point(ppos, pi, p, s0.val(), s1.val(), s2.val(), micro ? bt[pb].fMicro : bt[pb].fStep, cx, cy, cz, Lx, Ly,
-			Lz, nullptr);
+	if (S != 1) break;                            // only the odd movers' launch strides
+	wave_lds_sync();
+	}
 }
 
 // =====================================================================
@@ -2125,7 +2203,7 @@ __global__ __launch_bounds__(256) void k_cut_sorted(const float *__restrict__ th
 }
 
 // Device-side move-loop bookkeeping: ml[0] step stamp, ml[1] active count,
-// ml[2] count after the prune.  Everything a block of steps launches reads
+// ml[2] count after the prune, ml[3] odd movers of the block.  Everything a block of steps launches reads
 // these, so the block can be replayed as one graph with no host round trip.
 __global__ void k_ml_set(int *ml, int i, int v) { ml[i] = v; }
 __global__ void k_bump(int *ml) { ml[0] += 1; }
@@ -2202,7 +2280,7 @@ __global__ __launch_bounds__(1024) void k_prune_small(int *list, int *ml, const 
 	} else if (tid == 0) {
 		bact[0] = total;
 	}
-	if (tid == 0) { ml[1] = total; ml[2] = total; pin[1] = total; pin[4] = liveTotal[0]; }
+	if (tid == 0) { ml[1] = total; ml[2] = total; ml[3] = 0; pin[1] = total; pin[4] = liveTotal[0]; }
 }
 
 // Larger lists: flags with per-256 counts, a one-workgroup scan of the counts,
@@ -2286,7 +2364,7 @@ __global__ void k_copy_list(const int *__restrict__ in, int *ml, int *out, const
 	const int n = ml[2];
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < n) { out[i] = in[i]; box_count(in, n, mbox, i, bact); }
-	if (i == 0) { ml[1] = n; pin[1] = n; pin[4] = liveTotal[0]; }
+	if (i == 0) { ml[1] = n; ml[3] = 0; pin[1] = n; pin[4] = liveTotal[0]; }
 }
 
 __global__ void k_compact(const int *__restrict__ list, const int *__restrict__ flag,
@@ -2438,7 +2516,7 @@ extern "C" int skg_destroy(skg_ctx *c) {
 	skg_free_tree(&c->ts); skg_free_tree(&c->te); skg_free_tree(&c->tfull); skg_free_tree(&c->tfof);
 	dfree(&c->e_b2); dfree(&c->e_pos); dfree(&c->e_aux); dfree(&c->e_org); dfree(&c->e_code); dfree(&c->e_rho); dfree(&c->e_src); dfree(&c->e_live); dfree(&c->e_hit);
 	dfree(&c->e_box);
-	dfree(&c->m_pos); dfree(&c->m_old); dfree(&c->m_ord); dfree(&c->m_list); dfree(&c->m_list2); dfree(&c->m_box); dfree(&c->m_wrap);
+	dfree(&c->m_pos); dfree(&c->m_old); dfree(&c->m_ord); dfree(&c->m_list); dfree(&c->m_list2); dfree(&c->m_box); dfree(&c->m_wrap); dfree(&c->m_odd);
 	dfree(&c->tl_list); dfree(&c->tl_cnt);
 	skg_drop_graph(c);
 	dfree(&c->d_ml); dfree(&c->m_flag); dfree(&c->m_bcnt);
@@ -2597,7 +2675,7 @@ static int cover_launch(skg_ctx *c, int mode, float4 *ppos, const int *plist, in
 	k_cover<M_, C_><<<nb, SKG_TILE_T, 0, c->st>>>(ppos, plist, np, c->e_pos, c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, \
 			c->te.hi, c->te.nLeaf2, c->te.B, out, c->e_hit, stamp, nullptr, c->nBox > 1 ? pbox : nullptr, c->d_bt, micro, \
 			C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart, nullptr, nullptr, c->tlCap, nullptr, nullptr, 0, \
-			nullptr, out_dl, nullptr, nullptr, 1, 0)
+			nullptr, out_dl, nullptr, nullptr, 1, 0, nullptr, nullptr)
 #define CS(M_, C_)                                                                             \
 	k_cover_wave<M_, C_, 16><<<nblk(64L * np, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(ppos, plist, np, c->e_pos, \
 			c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, out, c->e_hit, stamp,       \
@@ -2840,7 +2918,7 @@ static void enqueue_lists(skg_ctx *c, long cap, int nsteps, int micro) {
 		k_tile_lists<<<nblk(cap, SKG_TILE_T), SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_list, (int)cap, c->e_pos, c->e_aux,
 				c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, c->te.lstart, pbox, c->d_bt, micro,
 				1.02f * (nsteps - 1), mabs, c->P.bPeriodic, 1.02f * (nsteps - 2), C[0], C[1], C[2], L[0], L[1], L[2],
-				c->tlCap, c->tl_list, c->tl_cnt, c->d_ml + 1, c->m_wrap);
+				c->tlCap, c->tl_list, c->tl_cnt, c->d_ml + 1, c->m_wrap, c->m_odd, c->d_ml + 3);
 }
 
 // nsteps Denmax steps over the active list (at most cap movers).
@@ -2862,6 +2940,7 @@ static int enqueue_steps(skg_ctx *c, long cap, bool sub, bool lists, int nsteps,
 	// refit a block of five steps over a small list is 8 launches (31 before),
 	// a whole pass 10.7 -> 8.7 ms for 2,048 points and 19.4 -> 16.5 for 32,768.
 	const bool lazy = fusedThr && c->cutReady && !bInitial && nsteps <= SKG_BLOCK_STEPS;
+	const bool elists = lists && c->useLists != 2;
 	if (lists) {
 		const int bslot = capturing ? -1 : skg_prof_begin(c);
 		enqueue_lists(c, cap, nsteps, micro);
@@ -2894,7 +2973,15 @@ static int enqueue_steps(skg_ctx *c, long cap, bool sub, bool lists, int nsteps,
 				c->e_pos, c->e_aux, c->e_org, c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, nullptr, \
 				ehit, 0, bthr, pbox, c->d_bt, micro, C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart,           \
 				lists ? c->tl_list : nullptr, lists ? c->tl_cnt : nullptr, c->tlCap, c->d_ml + 1, c->d_ml,  \
-				c->useLists != 2, c->d_eblk, nullptr, lists ? c->m_wrap : nullptr, c->d_bslot, c->nBox, nCut)
+				c->useLists != 2, c->d_eblk, nullptr, lists ? c->m_wrap : nullptr, c->d_bslot, c->nBox, nCut, \
+				elists ? c->m_odd : nullptr, c->d_ml + 3)
+		// odd movers first: what k_cover flags in this step joins them for the next
+#define MO(C_)                                                                                                \
+		k_cover_wave<1, C_, 1><<<ODD_WG, SKG_TILE_T, 0, c->st>>>(c->m_pos, c->m_odd, 0, c->e_pos, c->e_aux, c->e_org, \
+				c->e_code, c->nE, c->te.lo, c->te.hi, c->te.nLeaf2, c->te.B, nullptr, ehit, 0, bthr, pbox, c->d_bt, micro, \
+				C[0], C[1], C[2], L[0], L[1], L[2], c->te.lstart, c->d_ml + 3, c->d_ml, nullptr, c->d_bslot, c->nBox, nCut)
+		if (elists) { if (comp) { MO(true); } else { MO(false); } }
+#undef MO
 		if (comp) { MV(true); } else { MV(false); }
 #undef MV
 		if (pslot >= 0)
@@ -3002,24 +3089,20 @@ extern "C" int skg_init_move(skg_ctx *c, int *nMove) {
 	drop_graph(c);
 	const size_t nbm = (size_t)nblk(std::max(nm, 1), 256);
 	if (dalloc(&c->m_ord, nm) || dalloc(&c->m_pos, nm) || dalloc(&c->m_old, nm) || dalloc(&c->m_list, nm) ||
-	    dalloc(&c->m_wrap, nm) ||
+	    dalloc(&c->m_wrap, nm) || dalloc(&c->m_odd, nm) ||
 	    dalloc(&c->m_list2, nm) || dalloc(&c->m_box, nm) || dalloc(&c->m_flag, nm) || dalloc(&c->m_bcnt, 2 * nbm))
 		return SKG_E_NOMEM;
 	if (!c->d_ml && dalloc(&c->d_ml, 4)) return SKG_E_NOMEM;
 	if (!c->h_pin && hipHostMalloc((void **)&c->h_pin, 32, hipHostMallocDefault) != hipSuccess) return SKG_E_NOMEM;
 	if (c->useLists && nm > c->subMax) {
 		const size_t nt = (size_t)nblk(nm, 64);
-		// Entity lists: a tile whose list outgrows tlCap walks the tree at
-		// every step of its block, at about three times the cost of scanning a
-		// list.  On 256 boxes of up to 2^19 points, 11% of the tiles' lists
-		// pass 1024 entries and almost none 8192, so the capacity is 8192
-		// within a budget of 16 GiB (and an eighth of the free device memory),
-		// and at least 1024.
+		// Entity lists: LIST_CAP entries a tile, less where 16 GiB (or an eighth
+		// of the free device memory) do not hold that, and at least 1024.
 		if (c->useLists == 1 && !c->tlCapFixed) {
 			size_t fr = 0, tot = 0;
 			if (hipMemGetInfo(&fr, &tot) != hipSuccess) fr = 0;
 			const size_t budget = std::min<size_t>((size_t)16 << 30, fr / 8);
-			c->tlCap = (int)std::max<size_t>(1024, std::min<size_t>(8192, budget / (4 * nt)) & ~(size_t)63);
+			c->tlCap = (int)std::max<size_t>(1024, std::min<size_t>(LIST_CAP, budget / (4 * nt)) & ~(size_t)63);
 		}
 		if (dalloc(&c->tl_list, nt * c->tlCap) || dalloc(&c->tl_cnt, nt)) return SKG_E_NOMEM;
 	}
@@ -3032,6 +3115,7 @@ extern "C" int skg_init_move(skg_ctx *c, int *nMove) {
 		return rc;
 	ml_set(c, 0, 0);
 	ml_set(c, 1, nm);
+	ml_set(c, 3, 0);
 	if ((rc = count_active(c, nm))) return rc;
 	SKG_HIP(hipStreamSynchronize(c->st));
 	if (nMove) *nMove = nm;
