@@ -639,6 +639,56 @@ int skg_copy_tree_leaves(skg_ctx *c, DevTree *dst, const DevTree *src) {
 }
 
 
+// ---- windows: which of up to 64 staged records a lane needs, as a bit mask.
+// A ball (or reach) of squared radius R around e holds the point p when
+//   e.p + (R - |e|^2)/2 > |p|^2/2
+// in coordinates relative to the tile's centre: three fma and a compare per
+// record and lane instead of nine operations and a branch, the compare's carry
+// shifted into the mask (the first record in the highest bit).  Rounding can
+// err by under 12 2^-24 (|e|^2 + |p|^2 + R); the bounds are widened by 4e-6 of
+// it (and an unordered compare passes), so the mask holds every record that the
+// exact test (cover_hit's) accepts; the few others are dropped there.
+__device__ __forceinline__ float4 win_record(const float4 &A, float R, const float4 &o) {
+	const float x = A.x - o.x, y = A.y - o.y, z = A.z - o.z, e2 = fmaf(x, x, fmaf(y, y, z * z));
+	return make_float4(x, y, z, R < 0.f ? -INFINITY : fmaf(4e-6f, e2 + R, 0.5f * (R - e2)));
+}
+__device__ __forceinline__ float4 win_point(const float4 &p, const float4 &o) {
+	const float x = p.x - o.x, y = p.y - o.y, z = p.z - o.z, p2 = fmaf(x, x, fmaf(y, y, z * z));
+	return make_float4(x, y, z, (0.5f - 4e-6f) * p2);
+}
+__device__ __forceinline__ void win_push(unsigned &m, const float4 &T, const float4 &w) {
+	const float t = fmaf(T.x, w.x, fmaf(T.y, w.y, fmaf(T.z, w.z, T.w)));
+	// m = 2 m + !(t <= w.w)
+	asm("v_cmp_nle_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(t), "v"(w.w) : "vcc");
+}
+// The masks of the 64 records at sT (padded with -inf past the end); the second
+// half is left empty when there are at most 32.
+__device__ __forceinline__ void win_masks(const float4 *sT, int cnt, const float4 &w, unsigned &m0, unsigned &m1) {
+	m0 = m1 = 0;
+#pragma unroll 8
+	for (int t = 0; t < 32; ++t) win_push(m0, sT[t], w);
+	if (cnt > 32) {
+#pragma unroll 8
+		for (int t = 32; t < 64; ++t) win_push(m1, sT[t], w);
+	}
+}
+__device__ __forceinline__ float uniform_f(float x) { return __int_as_float(uniform_int(__float_as_int(x))); }
+// The or of every lane's v, in every lane.
+__device__ __forceinline__ unsigned wave_or(unsigned v) {
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);      // quad_perm [1,0,3,2]
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);      // quad_perm [2,3,0,1]
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);     // row_half_mirror
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);     // row_mirror
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);    // row_bcast:15 into rows 1 and 3
+	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);    // row_bcast:31 into rows 2 and 3
+	return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ void wave_lds_sync() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // =====================================================================
 // kNN: one wavefront per block of 64 Morton-consecutive queries, one lane
 // per query.  Each lane keeps a bounded max-heap of packed (d2, iOrder) keys
@@ -866,61 +916,323 @@ __global__ __launch_bounds__(64 * W) void k_knn(
 		for (int s = 0; s < k; ++s) heap_out[(size_t)s * n + qi] = heap[s * 64 + lane];
 }
 
+// The same search for the compensated mode and up to 128 neighbours without the
+// heap: each lane keeps the k smallest squared distances sorted in registers
+// (r[K-1] the largest; K - k slots in front hold -1), and a distance goes in by
+// one median per slot, r[i] = med3(r[i-1], x, r[i]).  The heap held a wavefront
+// to 8 (k + 1) 64 bytes of LDS, that is one wavefront per SIMD at k = 64, each
+// waiting out five to seven dependent LDS round trips per insertion; here four
+// fit (k = 64; five at k <= 32) and an insertion waits for nothing.  The registers
+// hold r once only while every loop around the insertion is wave-uniform with one
+// exit (walk conditions and trip counts go through readfirstlane); otherwise
+// the compiler keeps a second copy and spills.
+// 1,048,576 points, k = 64: 14.8 -> 8.2 ms (the search 5, the members 3.2);
+// 2M, k = 32: 29.3 -> 15.6; 96 boxes of 512 to 12,000: 2.4 -> 2.2; one box of 2,048: 0.8 -> 0.9.  It issues vector instructions half of the time; the
+// rest is the walk's and the windows' latency at four wavefronts.
+//
+// Candidates come in windows of up to 64 (a leaf, staged in LDS): a lane marks
+// those that may beat its largest distance (win_masks' test, the lane's radius
+// in place of the ball's), then works through its own marks with the exact fp32
+// distance, so insertions run as often as the lane with the most marks needs.
+//
+// The indices are collected afterwards, the k-th distance known: a second visit
+// of the leaves that the search scanned (at most KNN_LEAVES kept, else a second
+// walk) takes every d2 < h2 and, of those at h2 exactly, the smallest iOrders
+// that complete k -- the k smallest (d2, iOrder) keys, the largest of them in slot
+// 0, and forms the density's gather half on the way.  More than one candidate
+// at h2 (exact ties) sends the wavefront through further passes that find the
+// last iOrder to take, eight a pass, and through the collection again.
+// The plain mode keeps the heap (its fp32 sums run in the heap's slot order), and
+// so does k > 128 (r alone would fill the registers of two wavefronts).
+#define KNN_LEAVES 256
+template <int K, bool PER, bool BATCH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K <= 32 ? 5 : K <= 64 ? 4 : 2))) void k_knn_reg(
+		const float4 *__restrict__ spos, const int *__restrict__ sord, int n,
+		const float4 *__restrict__ nlo, const float4 *__restrict__ nhi, int nLeaf2, int B, float L, int k,
+		float *__restrict__ ball2_out, float *__restrict__ rhoG, unsigned long long *__restrict__ heap_out,
+		const int *__restrict__ sbox, const DevBox *__restrict__ bt, float *__restrict__ dlnk_out) {
+	__shared__ float4 s_T[4][64], s_A[4][64];
+	__shared__ int s_O[4][64], s_stk[4][64], s_lv[4][KNN_LEAVES];
+	__shared__ float s_std[4][64];
+	const int lane = threadIdx.x & 63, wv = uniform_int(threadIdx.x >> 6);
+	const int base = (xcd_tile(blockIdx.x, gridDim.x) * 4 + wv) * 64;
+	if (base >= n) return;                        // no workgroup barrier in this kernel
+	float4 *sT = s_T[wv], *sA = s_A[wv];
+	int *sO = s_O[wv], *stk = s_stk[wv], *lv = s_lv[wv];
+	float *stkd = s_std[wv];
+	const int sd0 = max(0, base - SKG_KNN_SEED), sd1 = min(n, base + 64 + SKG_KNN_SEED);   // seeded range
+	const int qi = base + lane;
+	const bool valid = qi < n;
+	const float4 q = spos[valid ? qi : base];
+	int qb = 0;
+	unsigned boff = 0u, bn = 0xFFFFFFFFu;
+	if (BATCH) { qb = sbox[valid ? qi : base]; boff = (unsigned)bt[qb].off; bn = (unsigned)bt[qb].n; }
+	const int wb0 = BATCH ? uniform_int(wave_min_i(qb)) : 0, wb1 = BATCH ? uniform_int(wave_max_i(qb)) : 0;
+	const float hL = 0.5f * L;
+	const float3 blo = make_float3(uniform_f(wave_min(q.x)), uniform_f(wave_min(q.y)), uniform_f(wave_min(q.z)));
+	const float3 bhi = make_float3(uniform_f(wave_max(q.x)), uniform_f(wave_max(q.y)), uniform_f(wave_max(q.z)));
+	const float4 o = make_float4(uniform_f(__shfl(q.x, 32, 64)), uniform_f(__shfl(q.y, 32, 64)), uniform_f(__shfl(q.z, 32, 64)), 0.f);
+	float r[K];
+#pragma unroll
+	for (int i = 0; i < K; ++i) r[i] = i < K - k ? -1.f : INFINITY;
+	auto insert = [&](float x) {
+#pragma unroll
+		for (int i = K - 1; i > 0; --i)           // in place (a median left to the compiler keeps two copies of r)
+			asm("v_med3_f32 %0, %1, %2, %0" : "+v"(r[i]) : "v"(r[i - 1]), "v"(x));
+		asm("v_min_f32 %0, %1, %0" : "+v"(r[0]) : "v"(x));
+	};
+
+	// ---- the candidates' sequence: the seeded range, then the leaves of a walk
+	// (nearest child first) or of the kept list, 64 at a time
+	int sp = 0, ps = 0, pe = 0;                   // walk stack; pending candidates
+	bool skip = false, cb = false, ci = false, need = false;
+	float4 wlo = o, whi = o;                      // the leaf's box
+	float top = INFINITY;
+	// prepares the leaf of a node; false when no lane needs it
+	auto leaf = [&](int node) {
+		const int start = (node - nLeaf2) * B;
+		if (start >= n) return false;
+		const int cnt = min(B, n - start);
+		if (start >= sd0 && start + cnt <= sd1) return false;     // seeded range
+		const float4 lo = nlo[node], hi = nhi[node];
+		need = valid && (!BATCH || brange_has(hi.w, qb)) && point_box_d2<PER>(lo, hi, q.x, q.y, q.z, L) <= top;
+		if (!__any(need)) return false;
+		cb = BATCH && __any(need && !brange_is(hi.w, qb));
+		ci = PER && uniform_int(!(fmaxf(bhi.x - lo.x, hi.x - blo.x) < 0.999f * hL &&
+				fmaxf(bhi.y - lo.y, hi.y - blo.y) < 0.999f * hL &&
+				fmaxf(bhi.z - lo.z, hi.z - blo.z) < 0.999f * hL)) != 0;
+		wlo = lo; whi = hi;
+		ps = start; pe = start + cnt; skip = true;
+		return true;
+	};
+	auto walk = [&](float R2) {                       // the next leaf of the walk, or false
+		while (sp > 0) {
+			--sp;
+			const int node = uniform_int(stk[sp]);
+			if (uniform_f(stkd[sp]) > R2) continue;
+			if (node >= nLeaf2) { if (leaf(node)) { stk[63] = node; return true; } continue; }
+			const int c0 = 2 * node;
+			const float4 h0 = nhi[c0], h1 = nhi[c0 + 1];
+			const float d0 = box_box_d2<PER>(nlo[c0], h0, blo, bhi, L);
+			const float d1 = box_box_d2<PER>(nlo[c0 + 1], h1, blo, bhi, L);
+			const bool m0 = !BATCH || brange_meets(h0.w, wb0, wb1), m1 = !BATCH || brange_meets(h1.w, wb0, wb1);
+			const bool near0 = d0 <= d1;
+			const int nf = near0 ? c0 : c0 + 1;
+			const float dn = near0 ? d0 : d1, df = near0 ? d1 : d0;
+			const bool mn = near0 ? m0 : m1, mf = near0 ? m1 : m0;
+			if (mf && df <= R2) { stk[sp] = nf ^ 1; stkd[sp] = df; ++sp; }
+			if (mn && dn <= R2) { stk[sp] = nf; stkd[sp] = dn; ++sp; }
+		}
+		return false;
+	};
+	// one window: each lane's marked candidates to f(has, position and mass, iOrder, d2)
+	auto window = [&](auto f) {
+		const int start = ps, cnt = min(64, pe - ps);
+		ps += cnt;
+		const int j = start + lane;
+		const bool here = lane < cnt && !(skip && j >= sd0 && j < sd1);
+		float4 C = make_float4(0.f, 0.f, 0.f, 0.f), T = make_float4(0.f, 0.f, 0.f, -INFINITY);
+		if (here) {
+			C = spos[j];
+			const float x = C.x - o.x, y = C.y - o.y, z = C.z - o.z;
+			const float e2 = fmaf(x, x, fmaf(y, y, z * z));
+			T = make_float4(x, y, z, (4e-6f - 0.5f) * e2);
+			sA[lane] = C;
+			sO[lane] = sord[j];
+		}
+		sT[lane] = T;
+		const unsigned long long in = __builtin_amdgcn_ballot_w64(here);
+		wave_lds_sync();
+		// e.p - |e|^2/2 > (|p|^2 - top)/2, widened by 4e-6 of the squares, by
+		// 1e-35 for squares that underflow (a record on the query, top = 0) and, with
+		// images (whose rounding is relative to L), by 1e-6 L times the radius
+		float px = q.x - o.x, py = q.y - o.y, pz = q.z - o.z, lim = INFINITY;
+		if (PER && ci) {
+			// each lane tests its own image: the one nearest the middle of the
+			// window's box, of extent w.  A pair that needs another one is at least
+			// (L - w)/2 apart, so a radius under that misses none
+			if (!skip) {                              // seeded: the window's own box
+				wlo = make_float4(uniform_f(wave_min(here ? C.x : INFINITY)), uniform_f(wave_min(here ? C.y : INFINITY)), uniform_f(wave_min(here ? C.z : INFINITY)), 0.f);
+				whi = make_float4(uniform_f(wave_max(here ? C.x : -INFINITY)), uniform_f(wave_max(here ? C.y : -INFINITY)), uniform_f(wave_max(here ? C.z : -INFINITY)), 0.f);
+			}
+			auto image = [&](float a, float b, float m, float v, float &pv) {   // box [a, b], lane at v
+				const float d = v - 0.5f * (a + b);
+				if (d > hL) pv = (m - L);
+				else if (d < -hL) pv = (m + L);
+				lim = fminf(lim, 0.499f * L - 0.5f * (b - a));
+			};
+			image(wlo.x, whi.x, px, q.x, px);
+			image(wlo.y, whi.y, py, q.y, py);
+			image(wlo.z, whi.z, pz, q.z, pz);
+		}
+		const float p2 = fmaf(px, px, fmaf(py, py, pz * pz));
+		float thr = 0.5f * (p2 - top) - 4e-6f * (p2 + top) - 1e-35f;
+		if (PER && ci) {
+			const float h = __builtin_amdgcn_sqrtf(top);
+			thr -= 1e-6f * L * (h + __builtin_amdgcn_sqrtf(p2));
+			if (!(h < lim)) thr = NAN;
+		}
+		if (!(top < INFINITY)) thr = NAN;             // an unbounded lane takes every record
+		const float4 w = make_float4(px, py, pz, thr);
+		unsigned m0 = 0, m1 = 0;
+		{
+			int t = 0;
+			for (const int e = min(cnt, 32); t < e; t += 4)
+#pragma unroll
+				for (int u = 0; u < 4; ++u) win_push(m0, sT[t + u], w);
+			m0 <<= 32 - t;
+		}
+		if (cnt > 32) {
+			int t = 32;
+			for (; t < cnt; t += 4)
+#pragma unroll
+				for (int u = 0; u < 4; ++u) win_push(m1, sT[t + u], w);
+			m1 <<= 64 - t;
+		}
+		m0 = need ? m0 & __brev((unsigned)in) : 0u;
+		m1 = need ? m1 & __brev((unsigned)(in >> 32)) : 0u;
+		const int trips = uniform_int(wave_max_i(__popc(m0) + __popc(m1)));
+		for (int it = 0; it < trips; ++it) {
+			const bool has = (m0 | m1) != 0, first = m0 != 0;
+			const int b = __builtin_clz((first ? m0 : m1) | 1u), t = (first ? 0 : 32) + b;
+			const unsigned keep = ~(0x80000000u >> b);
+			m0 = first ? m0 & keep : m0;
+			m1 = first ? m1 : m1 & keep;
+			const float4 C = sA[t];
+			const int oj = sO[t];
+			float dx = fsub(q.x, C.x), dy = fsub(q.y, C.y), dz = fsub(q.z, C.z);
+			if (PER && ci) {
+				float l = L;                          // opaque: the images are not kept in registers
+				asm volatile("" : "+s"(l));
+				dx = img_delta<PER>(q.x, fsub(q.x, l), fadd(q.x, l), C.x, hL);
+				dy = img_delta<PER>(q.y, fsub(q.y, l), fadd(q.y, l), C.y, hL);
+				dz = img_delta<PER>(q.z, fsub(q.z, l), fadd(q.z, l), C.z, hL);
+			}
+			f(has && (!(BATCH && cb) || (unsigned)oj - boff < bn), C, oj, sq3(dx, dy, dz));
+		}
+		wave_lds_sync();                              // every lane has read this window
+	};
+	// the seeded range may hold any box and any image
+	auto seed = [&]() {
+		ps = sd0; pe = sd1;
+		skip = false; cb = BATCH; ci = PER; need = valid;
+	};
+
+	// ---- the k smallest squared distances
+	int nlv = 0;
+	auto take = [&](bool has, const float4 &, int, float d2) {
+		const bool ok = has && d2 < r[K - 1];
+		insert(ok ? d2 : INFINITY);
+	};
+	seed();
+	bool walking = false;
+	for (;;) {
+		if (ps >= pe) {
+			top = r[K - 1];
+			const float R2 = uniform_f(wave_max(valid ? top : 0.f));
+			if (!walking) { walking = true; stk[0] = 1; stkd[0] = 0.f; sp = 1; }
+			if (!walk(R2)) break;
+			if (nlv < KNN_LEAVES) lv[nlv] = uniform_int(stk[63]);
+			++nlv;
+		}
+		top = r[K - 1];
+		window(take);
+	}
+	const float h2 = r[K - 1];
+	top = h2;
+
+	// ---- the members: every d2 < h2, and at h2 the iOrders up to last
+	const float ih2 = (float)(4.0 / (double)h2);
+	const float fNorm = (float)(0.5 * M_1_PI * sqrt((double)ih2) * (double)ih2);
+	// with dlnk_out, the gather half of d rho / d ln nSmooth over the same pairs,
+	// from exact periodic separations, h = sqrt(fBall2)/2
+	const bool dl = dlnk_out != nullptr;
+	const float ih = dl ? 1.0f / (0.5f * sqrtf(h2)) : 0.f;
+	Sum<true> acc, dacc;
+	// with non-finite separations fewer than k may be found: such slots name the query
+	if (valid && !(h2 < INFINITY))
+		for (int s = 0; s < k; ++s) heap_out[(size_t)s * n + qi] = (unsigned long long)0x7F800000u << 32 | (unsigned)sord[qi];
+	int last = INT_MAX, less = 0, at = 0;         // members below h2; candidates at h2
+	auto each = [&](auto f) {                     // the leaves again, for f
+		seed();
+		walking = false;
+		const bool kept = nlv <= KNN_LEAVES;
+		const float R2 = uniform_f(wave_max(valid ? h2 : 0.f));
+		for (int v = 0;;) {
+			if (ps >= pe) {
+				if (kept) {
+					while (v < nlv && !leaf(uniform_int(lv[v]))) ++v;
+					if (v++ >= nlv) break;
+				} else {
+					if (!walking) { walking = true; stk[0] = 1; stkd[0] = 0.f; sp = 1; }
+					if (!walk(R2)) break;
+				}
+			}
+			window(f);
+		}
+	};
+	for (int pass = 0; pass < 2; ++pass) {
+		acc.init(); dacc.init();
+		less = at = 0;
+		each([&](bool has, const float4 &C, int oj, float d2) {
+			const bool in = has && (d2 < h2 || (d2 == h2 && oj <= last));
+			if (!__any(in)) return;
+			float d2x = d2;
+			if (PER && ci) {
+				// weights from exact periodic separations (membership stays the
+				// reference's d2 test, so the neighbour set is unchanged)
+				float dx = fsub(q.x, C.x), dy = fsub(q.y, C.y), dz = fsub(q.z, C.z);
+				if (fabsf(dx) > hL || fabsf(dy) > hL || fabsf(dz) > hL) {
+					dx = exact_delta(q.x, C.x, dx > hL ? -L : (dx < -hL ? L : 0.f));
+					dy = exact_delta(q.y, C.y, dy > hL ? -L : (dy < -hL ? L : 0.f));
+					dz = exact_delta(q.z, C.z, dz > hL ? -L : (dz < -hL ? L : 0.f));
+					d2x = sq3(dx, dy, dz);
+				}
+			}
+			if (!in) return;
+			const unsigned long long key = ((unsigned long long)__float_as_uint(d2) << 32) | (unsigned)oj;
+			// the head: with one candidate at h2 that one, else the last
+			const bool head = d2 == h2 && (pass == 0 || oj == last);
+			if (d2 < h2) ++less;
+			else if (pass == 0 || !head) ++at;
+			if (head) { heap_out[qi] = key; return; }
+			acc.add(fmul(m4_term_f32(d2x, ih2, fNorm), C.w));
+			if (dl) dacc.add(dlnk_term(sqrtf(d2x), ih, C.w));
+			// members fill the slots from 1 up, the ones at h2 from k - 1 down
+			const int s = d2 < h2 ? less : k - at;
+			if (s > 0 && s < k) heap_out[(size_t)s * n + qi] = key;
+		});
+		if (pass || !__any(valid && at != 1)) break;
+		// ties at h2: the (k - less)-th smallest iOrder there, eight a pass
+		const int want = k - less;
+		last = -1;
+		for (int got = 0; __builtin_amdgcn_ballot_w64(valid && got < want); got += 8) {
+			int e[8];
+#pragma unroll
+			for (int i = 0; i < 8; ++i) e[i] = INT_MAX;
+			each([&](bool has, const float4 &, int oj, float d2) {
+				const int x = has && d2 == h2 && oj > last ? oj : INT_MAX;
+#pragma unroll
+				for (int i = 7; i > 0; --i) e[i] = max(min(e[i], x), e[i - 1]);
+				e[0] = min(e[0], x);
+			});
+			const int left = min(want - got, 8);
+#pragma unroll
+			for (int i = 0; i < 8; ++i) if (i < left) last = e[i];
+		}
+	}
+	if (!valid) return;
+	ball2_out[qi] = h2;
+	rhoG[qi] = acc.val();
+	if (dl) dlnk_out[qi] = dacc.val() * (float)(-M_1_PI / 6.0) * ih * ih * ih;
+}
+
 // =====================================================================
 // Ball cover: for each point, every entity whose ball strictly holds it
 // (non-periodic; periodic images are explicit replica entities, as the
 // reference's smx->pp).  MODE 0 accumulates the scatter half of the density,
 // MODE 1 the density gradient and then moves the point (kdMoveParticles).
 // =====================================================================
-// ---- windows: which of up to 64 staged records a lane needs, as a bit mask.
-// A ball (or reach) of squared radius R around e holds the point p when
-//   e.p + (R - |e|^2)/2 > |p|^2/2
-// in coordinates relative to the tile's centre: three fma and a compare per
-// record and lane instead of nine operations and a branch, the compare's carry
-// shifted into the mask (the first record in the highest bit).  Rounding can
-// err by under 12 2^-24 (|e|^2 + |p|^2 + R); the bounds are widened by 4e-6 of
-// it (and an unordered compare passes), so the mask holds every record that the
-// exact test (cover_hit's) accepts; the few others are dropped there.
-__device__ __forceinline__ float4 win_record(const float4 &A, float R, const float4 &o) {
-	const float x = A.x - o.x, y = A.y - o.y, z = A.z - o.z, e2 = fmaf(x, x, fmaf(y, y, z * z));
-	return make_float4(x, y, z, R < 0.f ? -INFINITY : fmaf(4e-6f, e2 + R, 0.5f * (R - e2)));
-}
-__device__ __forceinline__ float4 win_point(const float4 &p, const float4 &o) {
-	const float x = p.x - o.x, y = p.y - o.y, z = p.z - o.z, p2 = fmaf(x, x, fmaf(y, y, z * z));
-	return make_float4(x, y, z, (0.5f - 4e-6f) * p2);
-}
-__device__ __forceinline__ void win_push(unsigned &m, const float4 &T, const float4 &w) {
-	const float t = fmaf(T.x, w.x, fmaf(T.y, w.y, fmaf(T.z, w.z, T.w)));
-	// m = 2 m + !(t <= w.w)
-	asm("v_cmp_nle_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(t), "v"(w.w) : "vcc");
-}
-// The masks of the 64 records at sT (padded with -inf past the end); the second
-// half is left empty when there are at most 32.
-__device__ __forceinline__ void win_masks(const float4 *sT, int cnt, const float4 &w, unsigned &m0, unsigned &m1) {
-	m0 = m1 = 0;
-#pragma unroll 8
-	for (int t = 0; t < 32; ++t) win_push(m0, sT[t], w);
-	if (cnt > 32) {
-#pragma unroll 8
-		for (int t = 32; t < 64; ++t) win_push(m1, sT[t], w);
-	}
-}
-// The or of every lane's v, in every lane.
-__device__ __forceinline__ unsigned wave_or(unsigned v) {
-	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);      // quad_perm [1,0,3,2]
-	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);      // quad_perm [2,3,0,1]
-	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);     // row_half_mirror
-	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);     // row_mirror
-	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);    // row_bcast:15 into rows 1 and 3
-	v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);    // row_bcast:31 into rows 2 and 3
-	return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-__device__ __forceinline__ void wave_lds_sync() {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Whether a record whose w is w (the density, +inf for 0) is cut at threshold t.
 __device__ __forceinline__ bool cut_by(float w, float t) { return t > 0.f && (w < t || w == INFINITY); }
 
@@ -2646,9 +2958,22 @@ static void launch_knn(skg_ctx *c, bool per, bool comp) {
 	k_knn<KMAX, P_, C_, BATCH, W><<<nb, 64 * W, 0, c->st>>>(c->s_pos, c->s_ord, c->nS, c->ts.lo, c->ts.hi, \
 			c->ts.nLeaf2, c->ts.B, L, c->P.nSmooth, c->s_inv, c->s_ball2, c->s_rhoG, c->s_heap, \
 			c->s_box, c->d_bt, c->wantDlnk ? c->s_dlnkG : nullptr)
-	if (per) { if (comp) KL(true, true); else KL(true, false); }
-	else { if (comp) KL(false, true); else KL(false, false); }
+	if constexpr (KMAX > 128) {                   // up to 128 the compensated mode runs k_knn_reg
+		if (comp) { if (per) KL(true, true); else KL(false, true); return; }
+	}
+	if (per) KL(true, false); else KL(false, false);
 #undef KL
+}
+template <int K>
+static void launch_knn_reg(skg_ctx *c, bool per) {
+	const int nb = nblk(c->nS, 256);
+	const float L = per ? c->P.fPeriod[0] : FLT_MAX;
+#define KR(P_, B_)                                                                           \
+	k_knn_reg<K, P_, B_><<<nb, 256, 0, c->st>>>(c->s_pos, c->s_ord, c->nS, c->ts.lo, c->ts.hi, c->ts.nLeaf2, c->ts.B, L, \
+			c->P.nSmooth, c->s_ball2, c->s_rhoG, c->s_heap, c->s_box, c->d_bt, c->wantDlnk ? c->s_dlnkG : nullptr)
+	if (c->nBox > 1) { if (per) KR(true, true); else KR(false, true); }
+	else { if (per) KR(true, false); else KR(false, false); }
+#undef KR
 }
 // knnWaves: wavefronts per kNN workgroup (1 or 2; 2 only up to k = 64, where
 // two heaps fit a workgroup's LDS at useful occupancy)
@@ -2748,7 +3073,11 @@ extern "C" int skg_density(skg_ctx *c, float *fBall2, float *rho, int *nExtraSca
 		if (dalloc(&c->s_heap, (size_t)nS * k)) return SKG_E_NOMEM;
 		const bool comp = c->P.accumulate == SKG_ACC_COMPENSATED;
 		const int pslot = skg_prof_begin(c);
-		if (k <= 32) launch_knn<32>(c, per, comp);
+		// the plain mode's fp32 sums run in the heap's slot order, so it keeps the heap
+		if (comp && k <= 32) launch_knn_reg<32>(c, per);
+		else if (comp && k <= 64) launch_knn_reg<64>(c, per);
+		else if (comp && k <= 128) launch_knn_reg<128>(c, per);
+		else if (k <= 32) launch_knn<32>(c, per, comp);
 		else if (k <= 64) launch_knn<64>(c, per, comp);
 		else if (k <= 128) launch_knn<128>(c, per, comp);
 		else launch_knn<256>(c, per, comp);
