@@ -93,6 +93,32 @@ __device__ __forceinline__ float wrap_rel(float d, float L) {   // kd.c:1033-103
 	return d;
 }
 
+// The members s .. e-1 of a group, 64 apart per lane and in order: the records
+// of MEM_AHEAD rounds are loaded before the first of them is added (the lane's sums
+// are a serial chain; with one round's gather in flight at a time a wavefront
+// waits a memory round trip per 64 members).  A group of 250,000: 4.6 -> 1.6 ms;
+// 50,000: 0.64 -> 0.23.  load(o) gives the record of
+// member o, add(record) takes them in order.
+#define MEM_AHEAD 8
+template <typename Load, typename Add>
+__device__ __forceinline__ void each_member(const int *__restrict__ mem, int s, int e, int lane, Load load, Add add) {
+	int t = s + lane;
+	for (; t + (MEM_AHEAD - 1) * 64 < e; t += MEM_AHEAD * 64) {
+		int o[MEM_AHEAD];
+#pragma unroll
+		for (int u = 0; u < MEM_AHEAD; ++u) o[u] = mem[t + 64 * u];
+		decltype(load(0)) r[MEM_AHEAD];
+#pragma unroll
+		for (int u = 0; u < MEM_AHEAD; ++u) r[u] = load(o[u]);
+#pragma unroll
+		for (int u = 0; u < MEM_AHEAD; ++u) add(r[u]);
+	}
+	for (; t < e; t += 64) add(load(mem[t]));
+}
+struct MemberRec {
+	float m, x, y, z, vx, vy, vz;
+};
+
 // One wavefront per group g >= 1: mass, reference point (the member with the
 // largest iOrder), density centre of the moved positions and mass-weighted
 // velocity (kd.c:990-1059).
@@ -108,16 +134,16 @@ __global__ __launch_bounds__(64) void k_centers(const int *__restrict__ gs, cons
 	const float rx = pos[3 * last], ry = pos[3 * last + 1], rz = pos[3 * last + 2];
 	Acc am, ax, ay, az, vx, vy, vz;
 	am.init(); ax.init(); ay.init(); az.init(); vx.init(); vy.init(); vz.init();
-	for (int t = s + lane; t < e; t += 64) {
-		const int o = mem[t];
-		const float m = mass[o];
+	each_member(mem, s, e, lane, [&](int o) {
 		const float4 p = mpos[o];
-		am.add(m);
-		ax.add(wrap_rel(fsub(p.x, rx), Lx));
-		ay.add(wrap_rel(fsub(p.y, ry), Ly));
-		az.add(wrap_rel(fsub(p.z, rz), Lz));
-		vx.add(fmul(m, vel[3 * o])); vy.add(fmul(m, vel[3 * o + 1])); vz.add(fmul(m, vel[3 * o + 2]));
-	}
+		return MemberRec{mass[o], p.x, p.y, p.z, vel[3 * o], vel[3 * o + 1], vel[3 * o + 2]};
+	}, [&](const MemberRec &r) {
+		am.add(r.m);
+		ax.add(wrap_rel(fsub(r.x, rx), Lx));
+		ay.add(wrap_rel(fsub(r.y, ry), Ly));
+		az.add(wrap_rel(fsub(r.z, rz), Lz));
+		vx.add(fmul(r.m, r.vx)); vy.add(fmul(r.m, r.vy)); vz.add(fmul(r.m, r.vz));
+	});
 	float v[7] = {am.s, ax.s, ay.s, az.s, vx.s, vy.s, vz.s};
 	float w[7] = {am.c, ax.c, ay.c, az.c, vx.c, vy.c, vz.c};
 	for (int k = 0; k < 7; ++k) {
@@ -1683,6 +1709,10 @@ __global__ void k_compact_rec(const T *__restrict__ in, T *out, int nG, const in
 	int g = blockIdx.x * blockDim.x + threadIdx.x;
 	if (g < nG && g > 0 && keep[g]) out[off[g] + 1] = in[g];
 }
+// Largest distance from the centre per group.  Bound by the atomics on a large
+// group's one word; a particle that the word's current value already covers
+// sends none (the value only grows, so a stale read is a lower bound).
+// 2,097,152 particles, largest group 250,000: 2.8 -> 0.66 ms.
 __global__ void k_radius(const int *__restrict__ grp, int n, const float *__restrict__ pos,
 		const float4 *__restrict__ gcen, float Lx, float Ly, float Lz, unsigned *rad) {
 	int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1693,7 +1723,8 @@ __global__ void k_radius(const int *__restrict__ grp, int n, const float *__rest
 	float dx = wrap_rel(fsub(pos[3 * i], c.x), Lx), dy = wrap_rel(fsub(pos[3 * i + 1], c.y), Ly);
 	float dz = wrap_rel(fsub(pos[3 * i + 2], c.z), Lz);
 	float r = (float)sqrt((double)sq3(dx, dy, dz));
-	atomicMax(&rad[g], __float_as_uint(r));
+	if (__float_as_uint(r) > __hip_atomic_load(&rad[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+		atomicMax(&rad[g], __float_as_uint(r));
 }
 
 __global__ void k_gather_pos_members(const int *__restrict__ mem, int n, const float *__restrict__ pos,
@@ -2325,15 +2356,15 @@ __global__ __launch_bounds__(64) void k_group_com(const int *__restrict__ gs, co
 	const float rx = pos[3 * last], ry = pos[3 * last + 1], rz = pos[3 * last + 2];
 	Acc am, ax, ay, az, vx, vy, vz;
 	am.init(); ax.init(); ay.init(); az.init(); vx.init(); vy.init(); vz.init();
-	for (int t = s + lane; t < e; t += 64) {
-		const int o = mem[t];
-		const float m = mass[o];
-		am.add(m);
-		ax.add(fmul(m, wrap_rel(fsub(pos[3 * o], rx), Lx)));
-		ay.add(fmul(m, wrap_rel(fsub(pos[3 * o + 1], ry), Ly)));
-		az.add(fmul(m, wrap_rel(fsub(pos[3 * o + 2], rz), Lz)));
-		vx.add(fmul(m, vel[3 * o])); vy.add(fmul(m, vel[3 * o + 1])); vz.add(fmul(m, vel[3 * o + 2]));
-	}
+	each_member(mem, s, e, lane, [&](int o) {
+		return MemberRec{mass[o], pos[3 * o], pos[3 * o + 1], pos[3 * o + 2], vel[3 * o], vel[3 * o + 1], vel[3 * o + 2]};
+	}, [&](const MemberRec &r) {
+		am.add(r.m);
+		ax.add(fmul(r.m, wrap_rel(fsub(r.x, rx), Lx)));
+		ay.add(fmul(r.m, wrap_rel(fsub(r.y, ry), Ly)));
+		az.add(fmul(r.m, wrap_rel(fsub(r.z, rz), Lz)));
+		vx.add(fmul(r.m, r.vx)); vy.add(fmul(r.m, r.vy)); vz.add(fmul(r.m, r.vz));
+	});
 	float v[7] = {am.s, ax.s, ay.s, az.s, vx.s, vy.s, vz.s};
 	float w[7] = {am.c, ax.c, ay.c, az.c, vx.c, vy.c, vz.c};
 	for (int k = 0; k < 7; ++k) {
