@@ -270,7 +270,9 @@ int skg_fof_points_noalloc(skg_ctx *ctx, int n, const float *d_pos, float fTau, 
      SKG_TUNE_KNN       the kNN's shape: its tree's leaf size in
                         {8, 16, 32, 64} (independent of nBucket) and 1 or 2
                         wavefronts per kNN workgroup (each wavefront with its
-                        own 64 queries and LDS heaps; 2 only for nSmooth <= 64),
+                        own 64 queries and LDS heaps; 2 only for nSmooth <= 64;
+                        it has no effect on the compensated mode up to
+                        nSmooth 128, whose kNN keeps no heaps in LDS),
                         timed by the kNN stage of skg_density.
    Needs loaded particles; leaves the context loaded (stage of skg_load), so
    the caller runs the path again from skg_density.  Outputs (any may be
@@ -312,7 +314,7 @@ int skg_stage_times(skg_ctx *ctx, double *ms);
 #define SKG_K_UNB_POT 4      /* 20 flops per ordered pair */
 #define SKG_K_UNB_LOOP 5     /* removal loops of groups < 32768 members: 20 flops per kdSubPot pair */
 #define SKG_K_UNB_BIG 6      /* removal loops of larger groups (cooperative): 20 flops per kdSubPot pair */
-#define SKG_K_COVER_BUILD 7  /* a block's first move step building its entity lists: as SKG_K_COVER_MOVE */
+#define SKG_K_COVER_BUILD 7  /* the entity lists of a block's move steps: as SKG_K_COVER_MOVE */
 #define SKG_K_N 8
 int skg_set_profiling(skg_ctx *ctx, int on);
 /* Calibration copy (no reference counterpart): allocates two device buffers of
