@@ -1471,8 +1471,9 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_leaf_lists(const float4 *__restr
 // the block: the list then also holds what reaches the lane's image across that
 // face (with the full margin), and mwrap records the axis (1 + axis), so that a
 // crossing of that face leaves the list valid.  A lane near two or more faces
-// gets code 4, one near none 0: then any crossing sends its wavefront to the
-// tree walk.
+// gets code 4, one near none 0: then any crossing makes the mover odd, and the
+// rest of its tile keeps the list, which may hold entities that only the odd
+// mover needed (of another box, where the tile straddles two).
 #define WV_F 256              // nodes a wavefront's frontier holds
 #define TL_F 512              // the same of a tile: past it the tile is given up (2M gas+dark: 216 ms at 256, 179 at 512, 184 at 1024)
 #define WV_SIFT 32            // a longer frontier is tested against the points themselves
@@ -1768,8 +1769,11 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		const int *L = tlist + (size_t)tile * tcap;
 		const int wv = threadIdx.x >> 6;
 		float4 *sT = s_eT + wv * 64, *sA = s_eA + wv * LW, *sX = s_eX + wv * LW, *sO = s_eO + wv * LW;
-		// a tile that straddles boxes lists entities of each: a lane takes its own box's range
-		const bool straddle = pbox && __any(valid && pb != uniform_int(pb));
+		// a tile that straddles boxes lists entities of each: a lane takes its own
+		// box's range, and its own threshold.  Every mover of the tile counts, odd
+		// ones too: the list was built for all of them, and every lane stages
+		// entries (lanes past the end repeat the tile's first mover).
+		const bool straddle = pbox && __any(pb != uniform_int(pb));
 		const int elo = straddle ? eblk[pb] * 256 : 0, ehi = straddle ? eblk[pb + 1] * 256 : 0x7FFFFFFF;
 		const float4 o = make_float4(__shfl(p.x, 32, 64), __shfl(p.y, 32, 64), __shfl(p.z, 32, 64), 0.f);
 		const float4 w = win_point(p, o);
