@@ -6,6 +6,7 @@
 //   skg_move_first  main.c:395-404;  skg_move_block  main.c:410-416
 //   skg_microsteps  main.c:431-438
 #include "skg_common.h"
+#include "skg_hit.h"
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include <algorithm>
@@ -1774,6 +1775,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		// ones too: the list was built for all of them, and every lane stages
 		// entries (lanes past the end repeat the tile's first mover).
 		const bool straddle = pbox && __any(pb != uniform_int(pb));
+		const bool off = __any(far_off(p.x, p.y, p.z));
 		const int elo = straddle ? eblk[pb] * 256 : 0, ehi = straddle ? eblk[pb + 1] * 256 : 0x7FFFFFFF;
 		const float4 o = make_float4(__shfl(p.x, 32, 64), __shfl(p.y, 32, 64), __shfl(p.z, 32, 64), 0.f);
 		const float4 w = win_point(p, o);
@@ -1781,7 +1783,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		int en = lane < nl ? L[lane] : -1;
 		for (int c = 0; c < nl; c += LW) {
 			unsigned m[LW / 32];
-			bool reps = false;                        // a replica among the window's entries
+			bool reps = false, far = off;             // a replica, or a far position, among the window's entries
 #pragma unroll
 			for (int u = 0; u < LW / 64; ++u) {
 				m[2 * u] = m[2 * u + 1] = 0;
@@ -1797,6 +1799,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 				en = nx < nl ? L[nx] : -1;
 				if (!straddle && cut_by(X.w, cut)) X.x = -1.f;
 				sT[lane] = win_record(A, X.x, o);
+				far |= __any(far_off(A.x, A.y, A.z)) != 0;
 				A.w = __int_as_float(e);
 				sA[64 * u + lane] = A;
 				sX[64 * u + lane] = X;
@@ -1863,13 +1866,17 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 						}
 					}
 					float f = COMP ? grad_factor_f32(d2, X.y, X.z) : grad_factor(d2, X.y, X.z);
-					f = hit ? f : 0.f;
-					s0.add(fmul(dx, f)); s1.add(fmul(dy, f)); s2.add(fmul(dz, f));
+					if (GEN) {
+						s0.add(hit_term(hit, dx, f)); s1.add(hit_term(hit, dy, f)); s2.add(hit_term(hit, dz, f));
+					} else {                          // every separation is finite: one select, not three
+						f = hit ? f : 0.f;
+						s0.add(fmul(dx, f)); s1.add(fmul(dy, f)); s2.add(fmul(dz, f));
+					}
 					if (ehit && hit) ehit[__float_as_int(A.w)] = stamp;
 					hm = min(hm, hit ? __float_as_uint(X.w) : hm);
 				}
 			};
-			if (reps || straddle) work(std::true_type());
+			if (reps || straddle || far) work(std::true_type());
 			else work(std::false_type());
 			wave_lds_sync();                          // every lane has read this window
 		}
