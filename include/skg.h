@@ -271,8 +271,8 @@ int skg_fof_points_noalloc(skg_ctx *ctx, int n, const float *d_pos, float fTau, 
                         {8, 16, 32, 64} (independent of nBucket) and 1 or 2
                         wavefronts per kNN workgroup (each wavefront with its
                         own 64 queries and LDS heaps; 2 only for nSmooth <= 64;
-                        it has no effect on the compensated mode up to
-                        nSmooth 128, whose kNN keeps no heaps in LDS),
+                        not tried for the compensated mode up to nSmooth 128,
+                        whose kNN keeps no heaps in LDS),
                         timed by the kNN stage of skg_density.
    Needs loaded particles; leaves the context loaded (stage of skg_load), so
    the caller runs the path again from skg_density.  Outputs (any may be
@@ -284,10 +284,11 @@ int skg_fof_points_noalloc(skg_ctx *ctx, int n, const float *d_pos, float fTau, 
 #define SKG_TUNE_KNN      8
 #define SKG_TUNE_ALL      15
 int skg_autotune(skg_ctx *ctx, int what, int *nBucket, long long *subMax, int *potTile);
-/* The kNN shape in use: its tree's leaf size and wavefronts per kNN
-   workgroup (set by SKG_TUNE_KNN, or SKG_KNN_BUCKET / SKG_KNN_WAVES in the
-   environment at skg_create; default nBucket and 1).  No reference
-   counterpart. */
+/* The kNN shape in use: its tree's leaf size and wavefronts per workgroup of
+   the heap's search (set by SKG_TUNE_KNN, or SKG_KNN_BUCKET / SKG_KNN_WAVES in
+   the environment at skg_create; default nBucket and 1).  The compensated
+   mode up to nSmooth 128 searches in registers, where the wavefronts have no
+   effect and SKG_TUNE_KNN leaves them alone.  No reference counterpart. */
 int skg_knn_shape(skg_ctx *ctx, int *knnBucket, int *knnWaves);
 
 /* Per-stage device time in ms since skg_create, indexed by SKG_T_*. */

@@ -2986,8 +2986,13 @@ static void launch_knn_reg(skg_ctx *c, bool per) {
 	else { if (per) KR(true, false); else KR(false, false); }
 #undef KR
 }
-// knnWaves: wavefronts per kNN workgroup (1 or 2; 2 only up to k = 64, where
-// two heaps fit a workgroup's LDS at useful occupancy)
+// Whether the search runs in registers (k_knn_reg).  The plain mode's fp32 sums
+// run in the heap's slot order, so it keeps the heap.
+static bool knn_in_registers(const skg_ctx *c) {
+	return c->P.accumulate == SKG_ACC_COMPENSATED && c->P.nSmooth <= 128;
+}
+// knnWaves: wavefronts per workgroup of the heap's search (1 or 2; 2 only up to
+// k = 64, where two heaps fit a workgroup's LDS at useful occupancy)
 template <int KMAX>
 static void launch_knn(skg_ctx *c, bool per, bool comp) {
 	const bool two = KMAX <= 64 && c->knnWaves == 2;
@@ -3084,10 +3089,10 @@ extern "C" int skg_density(skg_ctx *c, float *fBall2, float *rho, int *nExtraSca
 		if (dalloc(&c->s_heap, (size_t)nS * k)) return SKG_E_NOMEM;
 		const bool comp = c->P.accumulate == SKG_ACC_COMPENSATED;
 		const int pslot = skg_prof_begin(c);
-		// the plain mode's fp32 sums run in the heap's slot order, so it keeps the heap
-		if (comp && k <= 32) launch_knn_reg<32>(c, per);
-		else if (comp && k <= 64) launch_knn_reg<64>(c, per);
-		else if (comp && k <= 128) launch_knn_reg<128>(c, per);
+		const bool reg = knn_in_registers(c);
+		if (reg && k <= 32) launch_knn_reg<32>(c, per);
+		else if (reg && k <= 64) launch_knn_reg<64>(c, per);
+		else if (reg) launch_knn_reg<128>(c, per);
 		else if (k <= 32) launch_knn<32>(c, per, comp);
 		else if (k <= 64) launch_knn<64>(c, per, comp);
 		else if (k <= 128) launch_knn<128>(c, per, comp);
@@ -3723,15 +3728,18 @@ extern "C" int skg_autotune(skg_ctx *c, int what, int *nBucket, long long *subMa
 	}
 	// 3. unbinding potential tile: timed on the groups of the next skg_unbind
 	if (what & SKG_TUNE_POT_TILE) c->tunePot = 1;
-	// 4. kNN shape: the kNN tree's leaf size and 1 or 2 wavefronts per kNN
-	// workgroup, timed by the tree and kNN stages of skg_density (best of two
-	// runs each, after one untimed run)
+	// 4. kNN shape: the kNN tree's leaf size and, for the heap's search, 1 or 2
+	// wavefronts per workgroup, timed by the tree and kNN stages of skg_density
+	// (best of two runs each, after one untimed run).  The search in registers
+	// has one workgroup shape: knnWaves stays as it is.
 	if (what & SKG_TUNE_KNN) {
 		double best = 1e300;
 		int bestB = c->knnBucket, bestW = c->knnWaves;
+		const int w0 = knn_in_registers(c) ? c->knnWaves : 1;
+		const int w1 = knn_in_registers(c) ? c->knnWaves : c->P.nSmooth <= 64 ? 2 : 1;
 		if ((rc = skg_density(c, nullptr, nullptr, nullptr))) return rc;
 		for (int B : {8, 16, 32, 64})
-			for (int W = 1; W <= (c->P.nSmooth <= 64 ? 2 : 1); ++W) {
+			for (int W = w0; W <= w1; ++W) {
 				c->knnBucket = B;
 				c->knnWaves = W;
 				double t = 1e300;
