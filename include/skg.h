@@ -260,8 +260,8 @@ int skg_fof_points_noalloc(skg_ctx *ctx, int n, const float *d_pos, float fTau, 
      SKG_TUNE_BUCKET    leaf size nBucket in {8, 16, 32, 64} (skg_density plus
                         the whole move loop per candidate);
      SKG_TUNE_MAPPING   the mover-to-lane mapping: the active count at and
-                        below which a block runs 16 lanes per mover instead of
-                        one lane per mover with its tiles' lists, from
+                        below which a block runs a wavefront per mover instead
+                        of one lane per mover with its tiles' lists, from
                         {2^14, 2^16, 2^18, 2^20}, each timed over the whole
                         move loop;
      SKG_TUNE_POT_TILE  the unbinding potential's workgroup / LDS tile in

@@ -141,17 +141,17 @@ struct skg_ctx {
 	size_t slotBytes[SKG_NSLOT] = {0};
 
 	// launch shapes (set at create; SKG_COVER_SUB_MAX overrides): point sets of
-	// at most subMax points use the sub-wave cover kernel
+	// at most subMax points take a wavefront each (k_cover_wave)
 	long subMax = 0;
 	int knnBucket = 0, knnWaves = 1;             // kNN tree leaf size (0: nBucket), wavefronts per workgroup of the heap's search
-	long s64Max = 0;            // at most this many active movers: 64 lanes (a wavefront) per mover
+	long s64Max = 0;            // at most this many active movers: their sums in the order of 64 lanes, above of 16
 	// per-tile lists of the current 5-step block: entities (SKG_TILE_LISTS=1,
 	// default), leaves (2) or none (0: every step walks the tree); tlCap
 	// entries per tile (a multiple of 4; for entity lists set from the mover
 	// count when the move loop starts, unless tlCapFixed)
 	int useLists = 1, tlCap = 1024, tlCapFixed = 0;
 	int *tl_list = nullptr, *tl_cnt = nullptr;
-	// device-resident move loop: ml[0] step stamp, ml[1] active, ml[2] next
+	// device-resident move loop: ml[0] step stamp, ml[1] active, ml[2] next, ml[3] odd movers
 	int *d_ml = nullptr;
 	int *m_flag = nullptr, *m_bcnt = nullptr;   // prune flags; block counts then offsets
 	int *m_wrap = nullptr;                       // per mover: wrapped across a periodic face since its tile's list was built

@@ -928,8 +928,10 @@ __global__ __launch_bounds__(64 * W) void k_knn(
 // exit (walk conditions and trip counts go through readfirstlane); otherwise
 // the compiler keeps a second copy and spills.
 // 1,048,576 points, k = 64: 14.8 -> 8.2 ms (the search 5, the members 3.2);
-// 2M, k = 32: 29.3 -> 15.6; 96 boxes of 512 to 12,000: 2.4 -> 2.2; one box of 2,048: 0.8 -> 0.9.  It issues vector instructions half of the time; the
-// rest is the walk's and the windows' latency at four wavefronts.
+// 2,097,152 of two species, k = 64: 29.3 -> 15.6; 96 boxes of 2,048 to 8,192,
+// k = 32: 2.4 -> 2.2; one box of 2,048: 0.8 -> 0.9 (32 wavefronts: one
+// wavefront's own time).  Its wavefronts issue 42% of their time and wait for
+// memory 41% (29,102,286 queries, k = 32).
 //
 // Candidates come in windows of up to 64 (a leaf, staged in LDS): a lane marks
 // those that may beat its largest distance (win_masks' test, the lane's radius
@@ -1244,7 +1246,7 @@ __device__ __forceinline__ bool cut_by(float w, float t) { return t > 0.f && (w 
 // stamps the hit entity (ehit) or keeps the lane's smallest positive density
 // among its hits (hmin; during the move loop the record's w holds the
 // entity's density, +inf for 0).
-template <int MODE, bool COMP, bool LAZYK = false>
+template <int MODE, bool COMP>
 __device__ __forceinline__ void cover_hit(int e, const float4 &A, const float4 &X, int K, bool want,
 		const float4 &p, const float4 *__restrict__ eorg, int *__restrict__ ehit, int stamp, float &hmin,
 		float Lx, float Ly, float Lz, Sum<COMP> &s0, Sum<COMP> &s1, Sum<COMP> &s2, bool dl = false,
@@ -1252,18 +1254,12 @@ __device__ __forceinline__ void cover_hit(int e, const float4 &A, const float4 &
 	float dx = fsub(A.x, p.x), dy = fsub(A.y, p.y), dz = fsub(A.z, p.z);
 	float d2 = sq3(dx, dy, dz);
 	if (want && d2 < X.x && !(MODE == 1 && cut_by(X.w, cut))) {
-		if (COMP || (MODE == 0 && dl)) {
-			// replica: separation from the source position plus the exact shift;
-			// LAZYK: the caller passes K < 0 and the code is read here, from the
-			// source record's w
-			float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
-			if (LAZYK && K < 0) { O = eorg[e]; K = (int)O.w; }
-			if (K != 13) {                       // 9(ix+1) + 3(iy+1) + (iz+1)
-				O = eorg[e];
-				dx = exact_delta(O.x, p.x, (float)(K / 9 - 1) * Lx);
-				dy = exact_delta(O.y, p.y, (float)((K / 3) % 3 - 1) * Ly);
-				dz = exact_delta(O.z, p.z, (float)(K % 3 - 1) * Lz);
-			}
+		if ((COMP || (MODE == 0 && dl)) && K != 13) {    // 9(ix+1) + 3(iy+1) + (iz+1)
+			// replica: separation from the source position plus the exact shift
+			const float4 O = eorg[e];
+			dx = exact_delta(O.x, p.x, (float)(K / 9 - 1) * Lx);
+			dy = exact_delta(O.y, p.y, (float)((K / 3) % 3 - 1) * Ly);
+			dz = exact_delta(O.z, p.z, (float)(K % 3 - 1) * Lz);
 		}
 		if (MODE == 0) {
 			s0.add(fmul(m4_w<COMP>(COMP ? sq3(dx, dy, dz) : d2, X.y, X.w), A.w));
@@ -1695,18 +1691,14 @@ __global__ __launch_bounds__(SKG_TILE_T) void k_tile_lists(const float4 *__restr
 	if (valid) odd[uniform_int(at) + lane] = pi;
 }
 
-// pbox (indexed like ppos; none: box 0) gives each point's box: a lane opens
-// only nodes holding its box, and the entity array starts every box on a new
-// leaf, so every entity a lane tests is of its own box.  MODE 1 takes the
-// box's step (micro: its micro-step).
-// List entries a wavefront holds in LDS at a time.  A longer window evens out
-// what the lanes have to do (13 hit rounds of 64 entries, 22 of 128), but its
-// LDS costs wavefronts: 128 measured 2% slower, 256 20%.
-#define LIST_W 64
 // Entries of a tile's list.  A longer one holds its launch: past it the tile's
 // movers get a wavefront each (48 boxes of 2,048 to 524,288 points, a pass:
 // 184 ms at 2048, 176 at 4096, 177 at 8192).
 #define LIST_CAP 4096
+// pbox (indexed like ppos; none: box 0) gives each point's box: a lane opens
+// only nodes holding its box, and the entity array starts every box on a new
+// leaf, so every entity a lane tests is of its own box.  MODE 1 takes the
+// box's step (micro: its micro-step).
 template <int MODE, bool COMP>
 __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_cover(
 		float4 *__restrict__ ppos, const int *__restrict__ plist, int np,
@@ -1722,9 +1714,8 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 	if (npDev) np = *npDev;                       // device-resident active count and step stamp
 	if (stampDev) stamp = *stampDev;
 	// staging slots for the entity-list scan, 64 per wavefront
-	constexpr int LW = MODE == 1 ? LIST_W : 64;
-	__shared__ float4 s_eA[SKG_TILE_T / 64 * LW], s_eX[SKG_TILE_T / 64 * LW];
-	__shared__ float4 s_eT[MODE == 1 ? SKG_TILE_T : 1], s_eO[MODE == 1 && COMP ? SKG_TILE_T / 64 * LW : 1];
+	__shared__ float4 s_eA[SKG_TILE_T], s_eX[SKG_TILE_T];
+	__shared__ float4 s_eT[MODE == 1 ? SKG_TILE_T : 1], s_eO[MODE == 1 && COMP ? SKG_TILE_T : 1];
 	__shared__ int s_eK[SKG_TILE_T];
 	const int lane = threadIdx.x & 63;
 	const int base = xcd_tile(blockIdx.x, gridDim.x) * SKG_TILE_T + (threadIdx.x & ~63);
@@ -1756,20 +1747,21 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 	if (nl >= 0 && !odd && mwrap && __any(valid && (mwrap[pi] & MWRAP_OUT) != 0)) nl = -1;
 	int node = nl >= 0 ? 0 : 1;
 	if (MODE == 1 && elist && nl > 0) {
-		// entity list (k_tile_lists): the listed entities in tree order, LIST_W
-		// at a time in this wavefront's slots of LDS (lane j gathers entry j's
-		// records).  Each lane first marks the entries its point may lie in
-		// (win_masks), then works through its own marks, lane by lane at
-		// different entries: the hit path runs as often as the lane with the
-		// most marks needs it, about 13 times for 64 entries, instead of once for
-		// each entry that some lane hits.  It has no branch: a lane without a
+		// entity list (k_tile_lists): the listed entities in tree order, 64 at a
+		// time in this wavefront's slots of LDS (lane j gathers entry j's records;
+		// windows of 128 or 256 even out the lanes' work, but their LDS costs
+		// wavefronts: 2% and 20% slower).  Each lane first marks the entries its
+		// point may lie in (win_masks), then works through its own marks, lane by
+		// lane at different entries: the hit path runs as often as the lane with
+		// the most marks needs it, about 13 times for 64 entries, instead of once
+		// for each entry that some lane hits.  It has no branch: a lane without a
 		// mark left, or whose entry the exact test drops, adds zeros (the sums
 		// start at +0, so that changes no bit).  The wavefront reads back only
 		// what it wrote itself, and LDS operations of one wavefront complete in
 		// order.
 		const int *L = tlist + (size_t)tile * tcap;
 		const int wv = threadIdx.x >> 6;
-		float4 *sT = s_eT + wv * 64, *sA = s_eA + wv * LW, *sX = s_eX + wv * LW, *sO = s_eO + wv * LW;
+		float4 *sT = s_eT + wv * 64, *sA = s_eA + wv * 64, *sX = s_eX + wv * 64, *sO = s_eO + wv * 64;
 		// a tile that straddles boxes lists entities of each: a lane takes its own
 		// box's range, and its own threshold.  Every mover of the tile counts, odd
 		// ones too: the list was built for all of them, and every lane stages
@@ -1781,76 +1773,46 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		const float4 w = win_point(p, o);
 		unsigned hm = __float_as_uint(INFINITY);      // hmin's bits (densities are >= 0)
 		int en = lane < nl ? L[lane] : -1;
-		for (int c = 0; c < nl; c += LW) {
-			unsigned m[LW / 32];
-			bool reps = false, far = off;             // a replica, or a far position, among the window's entries
-#pragma unroll
-			for (int u = 0; u < LW / 64; ++u) {
-				m[2 * u] = m[2 * u + 1] = 0;
-				if (c + 64 * u >= nl) continue;
-				const int e = en, nx = c + 64 * (u + 1) + lane;
-				float4 A = make_float4(0.f, 0.f, 0.f, 0.f), X = make_float4(-1.f, 0.f, 0.f, 0.f);
-				int K = 13;
-				if (e >= 0) {
-					A = epos[e];
-					X = eaux[e];
-					if (COMP) K = ecode[e];
-				}
-				en = nx < nl ? L[nx] : -1;
-				if (!straddle && cut_by(X.w, cut)) X.x = -1.f;
-				sT[lane] = win_record(A, X.x, o);
-				far |= __any(far_off(A.x, A.y, A.z)) != 0;
-				A.w = __int_as_float(e);
-				sA[64 * u + lane] = A;
-				sX[64 * u + lane] = X;
-				if (COMP) {
-					const unsigned long long b = __ballot(K != 13);
-					if (b) {                          // source positions and image codes
-						if (!reps && u > 0)
-							for (int v = 0; v < u; ++v) { float4 S = sA[64 * v + lane]; S.w = 13.f; sO[64 * v + lane] = S; }
-						reps = true;
-					}
-					if (reps) {
-						float4 S = A;
-						S.w = 13.f;
-						if (K != 13) S = eorg[e];
-						sO[64 * u + lane] = S;
-					}
-				}
-				wave_lds_sync();
-				win_masks(sT, nl - c - 64 * u, w, m[2 * u], m[2 * u + 1]);
-				wave_lds_sync();
+		for (int c = 0; c < nl; c += 64) {
+			const int e = en, nx = c + 64 + lane;
+			float4 A = make_float4(0.f, 0.f, 0.f, 0.f), X = make_float4(-1.f, 0.f, 0.f, 0.f);
+			int K = 13;
+			if (e >= 0) {
+				A = epos[e];
+				X = eaux[e];
+				if (COMP) K = ecode[e];
 			}
-			if (!valid)
-#pragma unroll
-				for (int u = 0; u < LW / 32; ++u) m[u] = 0;
+			en = nx < nl ? L[nx] : -1;
+			if (!straddle && cut_by(X.w, cut)) X.x = -1.f;
+			sT[lane] = win_record(A, X.x, o);
+			const bool far = off || __any(far_off(A.x, A.y, A.z));
+			A.w = __int_as_float(e);
+			sA[lane] = A;
+			sX[lane] = X;
+			const bool reps = COMP && __any(K != 13); // a replica among the window's entries
+			if (COMP && reps) {                       // source positions and image codes
+				float4 S = A;
+				S.w = 13.f;
+				if (K != 13) S = eorg[e];
+				sO[lane] = S;
+			}
+			wave_lds_sync();
+			unsigned m0, m1;
+			win_masks(sT, nl - c, w, m0, m1);
+			if (!valid) m0 = m1 = 0;
 			auto work = [&](auto general) {
 				constexpr bool GEN = decltype(general)::value;
-				for (;;) {
-					unsigned any = 0;
-#pragma unroll
-					for (int u = 0; u < LW / 32; ++u) any |= m[u];
-					if (!__any(any != 0)) break;
+				while (__any((m0 | m1) != 0)) {
 					// the lane's first mark, and the mark taken off
-					unsigned cur = m[LW / 32 - 1];
-					int b0 = LW - 32;
-#pragma unroll
-					for (int u = LW / 32 - 2; u >= 0; --u)
-						if (m[u]) { cur = m[u]; b0 = 32 * u; }
-					const int b = __builtin_clz(cur | 1u);
+					const bool has = (m0 | m1) != 0, first = m0 != 0;
+					const int b = __builtin_clz((first ? m0 : m1) | 1u), t = (first ? 0 : 32) + b;
 					const unsigned keep = ~(0x80000000u >> b);
-					bool before = true;
-#pragma unroll
-					for (int u = 0; u < LW / 32; ++u) {
-						const bool here = before && (m[u] != 0 || u == LW / 32 - 1);
-						m[u] = here ? m[u] & keep : m[u];
-						before = before && !here;
-					}
-					const int t = b0 + b;
+					m0 = first ? m0 & keep : m0;
+					m1 = first ? m1 : m1 & keep;
 					const float4 A = sA[t], X = sX[t];
 					float dx = fsub(A.x, p.x), dy = fsub(A.y, p.y), dz = fsub(A.z, p.z);
 					float d2 = sq3(dx, dy, dz);
-					bool hit = any != 0 && d2 < X.x;
+					bool hit = has && d2 < X.x;
 					if (GEN) {
 						const int e = __float_as_int(A.w);
 						hit = hit && e >= elo && e < ehi && !cut_by(X.w, cut);
@@ -1893,7 +1855,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		if (!__any(want)) continue;
 		const int2 rg = leaf_range(lstart, leaf, B, ne);
 		cover_scan_staged<MODE, COMP>(uniform_int(rg.x), uniform_int(rg.y - rg.x), want, p, epos, eaux, eorg, ecode,
-				ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x >> 6) * LW, s_eX + (threadIdx.x >> 6) * LW,
+				ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x & ~63), s_eX + (threadIdx.x & ~63),
 				s_eK + (threadIdx.x & ~63), lane, cut);
 	}
 	while (node) {
@@ -1905,8 +1867,8 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 		if (visit) {
 			const int2 rg = leaf_range(lstart, node - nLeaf2, B, ne);
 			cover_scan_staged<MODE, COMP>(uniform_int(rg.x), uniform_int(rg.y - rg.x), need, p, epos, eaux, eorg,
-					ecode, ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x >> 6) * LW,
-					s_eX + (threadIdx.x >> 6) * LW, s_eK + (threadIdx.x & ~63), lane, cut);
+					ecode, ehit, stamp, hmin, Lx, Ly, Lz, s0, s1, s2, dl, s_eA + (threadIdx.x & ~63),
+					s_eX + (threadIdx.x & ~63), s_eK + (threadIdx.x & ~63), lane, cut);
 		}
 		// next node in pre-order after node's subtree (strip trailing ones, step)
 		node = (node >> __builtin_ctz(~node)) + 1;
@@ -3701,8 +3663,8 @@ extern "C" int skg_autotune(skg_ctx *c, int what, int *nBucket, long long *subMa
 		}
 		c->P.nBucket = bestB;
 	}
-	// 2. mover mapping: the active count at and below which a block runs 16
-	// lanes per mover instead of one lane per mover (with its tiles' lists),
+	// 2. mover mapping: the active count at and below which a block runs a
+	// wavefront per mover instead of one lane per mover (with its tiles' lists),
 	// timed over the whole move loop for each candidate (a block's cost with
 	// lists includes its list build, which a single step on a subset misses)
 	if (what & SKG_TUNE_MAPPING) {
