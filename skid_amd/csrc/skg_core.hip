@@ -1785,7 +1785,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 			en = nx < nl ? L[nx] : -1;
 			if (!straddle && cut_by(X.w, cut)) X.x = -1.f;
 			sT[lane] = win_record(A, X.x, o);
-			const bool far = off || __any(far_off(A.x, A.y, A.z));
+			bool far = off || __any(far_off(A.x, A.y, A.z));
 			A.w = __int_as_float(e);
 			sA[lane] = A;
 			sX[lane] = X;
@@ -1795,13 +1795,14 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 				S.w = 13.f;
 				if (K != 13) S = eorg[e];
 				sO[lane] = S;
+				far |= __any(far_off(S.x, S.y, S.z)) != 0;
 			}
 			wave_lds_sync();
 			unsigned m0, m1;
 			win_masks(sT, nl - c, w, m0, m1);
 			if (!valid) m0 = m1 = 0;
-			auto work = [&](auto general) {
-				constexpr bool GEN = decltype(general)::value;
+			auto work = [&](auto general, auto unbounded) {
+				constexpr bool GEN = decltype(general)::value, FAR = decltype(unbounded)::value;
 				while (__any((m0 | m1) != 0)) {
 					// the lane's first mark, and the mark taken off
 					const bool has = (m0 | m1) != 0, first = m0 != 0;
@@ -1828,7 +1829,7 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 						}
 					}
 					float f = COMP ? grad_factor_f32(d2, X.y, X.z) : grad_factor(d2, X.y, X.z);
-					if (GEN) {
+					if (FAR) {
 						s0.add(hit_term(hit, dx, f)); s1.add(hit_term(hit, dy, f)); s2.add(hit_term(hit, dz, f));
 					} else {                          // every separation is finite: one select, not three
 						f = hit ? f : 0.f;
@@ -1838,8 +1839,9 @@ __global__ __launch_bounds__(SKG_TILE_T) __attribute__((amdgpu_waves_per_eu(8, 8
 					hm = min(hm, hit ? __float_as_uint(X.w) : hm);
 				}
 			};
-			if (reps || straddle || far) work(std::true_type());
-			else work(std::false_type());
+			if (far) work(std::true_type(), std::true_type());
+			else if (reps || straddle) work(std::true_type(), std::false_type());
+			else work(std::false_type(), std::false_type());
 			wave_lds_sync();                          // every lane has read this window
 		}
 		hmin = __uint_as_float(hm);

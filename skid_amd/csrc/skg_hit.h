@@ -14,9 +14,9 @@
 // value is unordered) and dropped by the exact test, and 0 d would be NaN.
 SKG_HIT_FN float hit_term(bool hit, float d, float f) { return hit ? d * f : 0.f; }
 
-// Whether a separation from this position can fail to be finite.  Where no
-// mover of the tile and no entry of the window lies so, a step multiplies by
-// zero instead: one select a mark, not three (the selects in every window cost
-// 0.9% of a pass of 2,097,152 particles of gas and dark matter, 1.3% of one of 48
-// uneven boxes).
-SKG_HIT_FN bool far_off(float x, float y, float z) { return !(fabsf(x) + fabsf(y) + fabsf(z) < 1e38f); }
+// Whether a separation from this position, with a period's shift, can fail to be
+// finite.  Where no mover of the tile and no entry of the window lies so, a step
+// multiplies by zero instead: one select a mark, not three (the selects in every
+// window cost 0.9% of a pass of 2,097,152 particles of gas and dark matter, 1.3%
+// of one of 48 uneven boxes).
+SKG_HIT_FN bool far_off(float x, float y, float z) { return !(fabsf(x) + fabsf(y) + fabsf(z) < 1e37f); }

@@ -64,12 +64,14 @@ def test_step_with_a_far_entry_equals_the_walk(hit_term):
 
 
 def test_near_positions_have_finite_separations(lib):
-    """No position that passes as near lies so far from another one that their separation overflows."""
-    edge = [0.0, 0.5, -0.5, 1e20, -1e20, 0.99e38, -0.99e38, 1.01e38, -3.4e38, np.inf, -np.inf, np.nan]
+    """No position that passes as near lies so far from another one that their separation overflows, nor its
+    sum with a period's shift (a replica and its source are near, so the shift is at most twice as far)."""
+    edge = [0.0, 0.5, -0.5, 1e20, -1e20, 0.99e37, -0.99e37, 1.01e37, -3.4e38, np.inf, -np.inf, np.nan]
     near = [np.float32(v) for v in edge if not lib.far(v, 0.0, 0.0)]
     assert len(near) == 7
     for a in near:
         for b in near:
             assert np.isfinite(a - b)
+            assert np.isfinite((a - b) + np.float32(2) * near[-2]) and np.isfinite((a - b) + np.float32(2) * near[-1])
     for v in edge[7:]:
         assert lib.far(v, 0, 0) and lib.far(0, v, 0) and lib.far(0, 0, v)
