@@ -316,7 +316,8 @@ extern "C" int skg_fof(skg_ctx *c, int *grp, int *nGroup) {
 	skg_timer_start(c);
 	k_zero<<<nblk(c->n, 256), 256, 0, c->st>>>(c->d_grp, c->n);
 	if (c->nMove > 0) {
-		if ((rc = fof_run(c, c->m_pos, c->nMove, c->P.fTau, c->m_ord, c->d_grp, &ng,
+		// one box: its own tau (several: each reads its tau beside its points)
+		if ((rc = fof_run(c, c->m_pos, c->nMove, c->hbox[0].tau, c->m_ord, c->d_grp, &ng,
 				c->nBox > 1 ? c->m_box : nullptr))) return rc;
 	}
 	skg_timer_stop(c, SKG_T_FOF);

@@ -1943,7 +1943,7 @@ extern "C" int skg_unbind(skg_ctx *c, int *nUnbound) {
 			if ((rc = skg_morton_sort(c, zp, nullptr, n0, perm, batch ? zb : nullptr))) return rc;
 			k_gather4g<<<nblk(n0, 256), 256, 0, c->st>>>(zp, ze, zb, perm, n0, zs, zes, zbs);
 			if ((rc = skg_build_tree(c, &t, zs, n0, c->P.nBucket, nullptr, batch ? zbs : nullptr))) return rc;
-			const float sc2 = c->P.fScoop * c->P.fScoop;
+			const float sc2 = c->hbox[0].scoop * c->hbox[0].scoop;   // one box (several: each its own)
 			k_unb_scoop<<<nG - 1, 64, 0, c->st>>>(G->gstart, G->gend, nG, G->cen, G->rel, zs, zes, n0, t.lo, t.hi,
 					t.nLeaf2, t.B, c->P.bPeriodic ? L[0] : FLT_MAX, c->P.bPeriodic, sc2, G->uq, G->uv, G->uphi,
 					c->P.G, c->P.iSoftType, nMax, batch ? zbs : nullptr, G->mem, c->d_boxOf, c->d_bt);
