@@ -11,6 +11,7 @@
 // as uniform loads); the energies, the per-group centre-of-mass updates and
 // the bound/unbound sign test run in fp64.
 #include "skg_common.h"
+#include "skg_seg.h"
 #include <hip/hip_cooperative_groups.h>
 #include <algorithm>
 #include <cfloat>
@@ -65,12 +66,15 @@ __global__ void k_izero(int *a, int n) {
 	int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < n) a[i] = 0;
 }
-__global__ void k_seg(const unsigned long long *__restrict__ key, int n, int *gs, int *ge) {
-	int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n) return;
-	int g = (int)(key[i] >> 32);
-	if (i == 0 || (int)(key[i - 1] >> 32) != g) gs[g] = i;
-	if (i == n - 1 || (int)(key[i + 1] >> 32) != g) ge[g] = i + 1;
+// gs[g], ge[g]: the segment of group g, one search per group (a group ends where
+// the next one starts).  Ids without members have empty segments in place, which
+// k_unb_setup's search over the starts needs.
+__global__ void k_seg(const unsigned long long *__restrict__ key, int n, int nG, int *gs, int *ge) {
+	int g = blockIdx.x * blockDim.x + threadIdx.x;
+	if (g > nG) return;
+	const int s = group_start(key, n, g);
+	if (g < nG) gs[g] = s;
+	if (g > 0) ge[g - 1] = s;
 }
 __global__ void k_count(const int *gs, const int *ge, int nG, int *cnt) {
 	int g = blockIdx.x * blockDim.x + threadIdx.x;
@@ -205,11 +209,8 @@ __global__ void k_unb_setup(const int *__restrict__ gs, const int *__restrict__ 
 		float hx, float hy, float hz, int nMax, float4 *uq, float4 *uv, float2 *uphi, int *uord, int nTot) {
 	int t = blockIdx.x * blockDim.x + threadIdx.x;
 	if (t >= nTot) return;
-	// locate the group by binary search over segment starts
-	int lo = 1, hi = nG - 1;
-	while (lo < hi) { int mid = (lo + hi + 1) >> 1; if (gs[mid] <= t) lo = mid; else hi = mid - 1; }
-	const int g = lo;
-	if (g < 1 || t < gs[g] || t >= ge[g]) return;
+	const int g = group_at(gs, ge, nG, t);
+	if (!g) return;
 	const int o = mem[t];
 	const float4 r = grel[g];
 	float dx = fsub(pos[3 * o], r.x), dy = fsub(pos[3 * o + 1], r.y), dz = fsub(pos[3 * o + 2], r.z);
@@ -1752,9 +1753,7 @@ static int group_sort(skg_ctx *c) {
 	if (skg_ensure_keys(c, n)) return SKG_E_NOMEM;
 	k_gkeys<<<nblk(n, 256), 256, 0, c->st>>>(c->d_grp, n, c->k64a, c->v32a);
 	if ((rc = skg_sort_pairs(c, c->k64a, c->k64b, c->v32a, G->mem, n, 64))) return rc;
-	k_izero<<<nblk(G->nG, 256), 256, 0, c->st>>>(G->gstart, G->nG);
-	k_izero<<<nblk(G->nG, 256), 256, 0, c->st>>>(G->gend, G->nG);
-	k_seg<<<nblk(n, 256), 256, 0, c->st>>>(c->k64b, n, G->gstart, G->gend);
+	k_seg<<<nblk((long)G->nG + 1, 256), 256, 0, c->st>>>(c->k64b, n, G->nG, G->gstart, G->gend);
 	k_count<<<nblk(G->nG, 256), 256, 0, c->st>>>(G->gstart, G->gend, G->nG, G->count);
 	SKG_HIP(hipGetLastError());
 	return 0;
